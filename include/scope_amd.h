@@ -467,6 +467,23 @@ int scope_attn_block_mass(const scope_attn_params* p, const uint16_t* q, const u
                           const float* delta_main, const float* width, float* lse, float* mass,
                           void* stream);
 
+/* The same masses and LSE in one pass over the scores, with a workspace of
+ * scope_attn_block_mass_workspace_bytes (at most 256 MiB, or one list row's
+ * bytes).  Every entry of mass is written: 0 for the blocks that a row does
+ * not list. */
+int64_t scope_attn_block_mass_workspace_bytes(const scope_attn_params* p);
+int scope_attn_block_mass_ws(const scope_attn_params* p, const uint16_t* q, const uint16_t* k,
+                             const int32_t* kv_num, const int32_t* kv_idx, const int32_t* docs,
+                             const int32_t* ds_tok_end, const void* table, const float* coeff_cos,
+                             const float* coeff_sin, const float* b0, const float* slope,
+                             const float* delta_main, const float* width, float* lse, float* mass,
+                             void* work, void* stream);
+
+/* The dense document-causal lists of the teacher's block mass: row (h, qb)
+ * lists the blocks ds_local[qb] .. qb (kv_num [H][NB], kv_idx [H][NB][NB],
+ * entries past a row's number repeat qb). */
+int scope_causal_lists(const int32_t* ds_local, int H, int NB, int32_t* kv_num, int32_t* kv_idx, void* stream);
+
 /* ------------------------------------------------------------------------
  * Decode: the attention of one new token (position t) against the KV cache,
  * over its q-block's listed key blocks with the document-causal mask.  No

@@ -116,6 +116,9 @@ _PROTOS = {
     "scope_spectral_table": (c_int, [c_int, P, c_int, c_int64, c_int, P, P]),
     "scope_attn_fwd": (c_int, [C.POINTER(AttnParams)] + [P] * 17),
     "scope_attn_block_mass": (c_int, [C.POINTER(AttnParams)] + [P] * 16),
+    "scope_attn_block_mass_workspace_bytes": (c_int64, [C.POINTER(AttnParams)]),
+    "scope_attn_block_mass_ws": (c_int, [C.POINTER(AttnParams)] + [P] * 17),
+    "scope_causal_lists": (c_int, [P, c_int, c_int, P, P, P]),
     "scope_attn_bwd_workspace_bytes": (c_int64, [C.POINTER(AttnParams)]),
     "scope_decode_workspace_bytes": (c_int64, [C.POINTER(DecodeParams)]),
     "scope_decode_attn": (c_int, [C.POINTER(DecodeParams)] + [P] * 10),

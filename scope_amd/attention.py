@@ -133,15 +133,10 @@ def teacher_block_mass(q: torch.Tensor, k: torch.Tensor, docs: torch.Tensor, *, 
 
     T = q.shape[-2]
     bs = block_size
-    NB = T // bs
     docs = docs.reshape(-1).to(torch.int32).contiguous()
     _, ds_local, ds_tok_end = ops.doc_starts(docs, bs)
     # dense document-causal list: key blocks from the q-block's first document start to the diagonal
-    qb = torch.arange(NB, device=q.device, dtype=torch.int32)
-    first = ds_local.to(torch.int32)
-    kv_num = (qb - first + 1)[None].expand(q.shape[1], -1).contiguous()
-    kv_idx = torch.minimum(first[:, None] + torch.arange(NB, device=q.device, dtype=torch.int32)[None],
-                           qb[:, None])[None].expand(q.shape[1], -1, -1).contiguous()
+    kv_num, kv_idx = ops.causal_lists(ds_local, q.shape[1])
     kw = dict(bias_mode="none")
     if spectral is not None:
         if spectral.offset != "token":

@@ -306,6 +306,11 @@ struct AttnArgs {
   float* delta;      // rowsum(dO∘O) [H,T]
   uint16_t* qfeat;   // token mode: query-side features [H,T][kTokRow] (hi g0, hi g1, lo g0, lo g1)
   float* mass;       // block mass [H,QB,NB] (forward mass pass)
+  // block mass in one pass: (maximum, sum of exponentials) of every list entry and row,
+  // [part_rows][maxkv][bs], for the list rows h·QB + qb from part_row0; a workgroup takes
+  // part_entries of a row's entries
+  float2* part;
+  int part_row0, part_rows, part_entries;
   const float* pair_bias;  // per-list-entry score bias [H,QB,maxkv] (natural log) or null
   float* dpair;            // backward: tile sums of dS per (key-block part, h, qb, entry) [P][H][QB][maxkv] or null
   // backward, no bias or block bias: the log2-domain softmax offset of every

@@ -31,6 +31,7 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -95,9 +96,11 @@ __device__ __forceinline__ void fwd_scores(const AttnArgs& a, const Tile& b, con
 }
 
 // What the forward kernel produces: the attention output and its LSE; the
-// LSE alone (no P·V); or, given the LSE, the probability mass of every
-// listed key block summed over the q-block's rows (no P·V either).
-enum FwdKind { kFwdAttn = 0, kFwdLse = 1, kFwdMass = 2 };
+// LSE alone (no P·V); given the LSE, the probability mass of every listed key
+// block summed over the q-block's rows (no P·V either); or, for a run of
+// list entries, every row's maximum and sum of exponentials per entry, from
+// which mass_merge_kernel forms the LSE and the masses.
+enum FwdKind { kFwdAttn = 0, kFwdLse = 1, kFwdMass = 2, kFwdPart = 3 };
 
 // Every mode runs two wavefronts per SIMD at either block size: for bs=128
 // the compiler would otherwise take up to 512 registers and run one (the
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
   constexpr int BN = 64;  // keys per staged tile
   constexpr int NSUB = BS / BN;
   constexpr bool TOK = MODE >= 2, GATE = MODE == 3;
-  constexpr bool MASS = KIND == kFwdMass, PV = KIND == kFwdAttn;
+  constexpr bool MASS = KIND == kFwdMass, PV = KIND == kFwdAttn, PART = KIND == kFwdPart;
   // bs=256 attention: wavefronts 4-7 run half a tile behind wavefronts 0-3
   // (see the loop below), which needs a third tile buffer
   constexpr bool STAGGER = PV && BS == 256;
@@ -130,8 +133,23 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid % 64, g = lane / 32, lr = lane % 32;
-  const int tile = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = tile / a.QB, qb = tile % a.QB;
+  int row, e0 = 0;  // list row and its first entry
+  if (PART) {
+    // Each XCD takes every eighth list row and walks the lists a run of entries
+    // at a time: its workgroups of the moment read the same key blocks from its
+    // L2, and the long and the short lists of a causal mask fall on all XCDs
+    // alike (with whole runs per XCD, the runs that every row has took three
+    // times the mean)
+    const int per = (a.part_rows + 7) / 8, x = blockIdx.x % 8, j = blockIdx.x / 8;
+    row = (j % per) * 8 + x;
+    if (row >= a.part_rows) return;
+    e0 = j / per * a.part_entries;
+    row += a.part_row0;
+    e0 = j / per * a.part_entries;
+  } else {
+    row = xcd_remap(blockIdx.x, gridDim.x);
+  }
+  const int h = row / a.QB, qb = row % a.QB;
   const int64_t q0 = static_cast<int64_t>(qb) * BS;
   const int wrow_lo = static_cast<int>(q0) + wave * 32;
   const int64_t hT = static_cast<int64_t>(h) * a.T;
@@ -139,12 +157,16 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
   R.row = wrow_lo + lr;
 
   const int64_t lrow = static_cast<int64_t>(h) * a.QB + qb;
-  const int n = min(a.kv_num[lrow], a.maxkv);  // maxkv <= kListLds
+  int n = min(a.kv_num[lrow], a.maxkv);  // maxkv <= kListLds
+  if (PART) {
+    if (e0 >= n) return;
+    n = min(n, e0 + a.part_entries);
+  }
   const int32_t* lst = a.kv_idx + lrow * a.maxkv;
-  for (int t = tid; t < min(n, kListLds); t += NT) kbs[t] = lst[t];
+  for (int t = e0 + tid; t < min(n, kListLds); t += NT) kbs[t] = lst[t];
   const bool pbias = a.pair_bias != nullptr;
   if (pbias)
-    for (int t = tid; t < min(n, kListLds); t += NT) kbias[t] = a.pair_bias[lrow * a.maxkv + t] * kLog2e;
+    for (int t = e0 + tid; t < min(n, kListLds); t += NT) kbias[t] = a.pair_bias[lrow * a.maxkv + t] * kLog2e;
   if (MASS)
     for (int t = tid; t < n * NW; t += NT) mslot[t] = 0.f;  // n <= kListLds (checked on the host)
 
@@ -192,6 +214,15 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
     for (int o2 = 32; o2 > 0; o2 >>= 1) pacc += __shfl_xor(pacc, o2, 64);
     if (lane == 0) mslot[pent * NW + wave] += pacc;
     pacc = 0.f;
+  };
+  // PART: the maximum (log2 units) and the sum of exponentials of list entry
+  // pent for the wavefront's 32 rows, l_run counting from the entry's first tile
+  auto part_flush = [&]() __attribute__((always_inline)) {
+    if (pent < 0) return;
+    const float l_ent = l_run + xor32(l_run);
+    if (g == 0)
+      a.part[((lrow - a.part_row0) * a.maxkv + pent) * BS + wave * 32 + lr] = make_float2(m_run, l_ent);
+    l_run = 0.f;
   };
   float lse2 = 0.f;  // mass: the row's LSE in log2 units
   if (MASS) lse2 = a.lse[hT + R.row] * kLog2e;
@@ -306,6 +337,10 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
       return false;
     }
 
+    if (PART && it / NSUB != pent) {  // the tiles of a list entry come in a row
+      part_flush();
+      pent = it / NSUB;
+    }
     // online softmax (log2 domain); the running maximum moves only by more than kLazy
     float mx = -INFINITY;
 #pragma unroll
@@ -331,6 +366,14 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
     const float off = m_run == -INFINITY ? -INFINITY : tconst - m_run;
 
     float psum = 0.f;
+    if constexpr (!PV) {
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) psum += __builtin_amdgcn_exp2f(fmaf(s[mb][r], csm, off));
+      l_run += psum;
+      return false;
+    }
     probs_half(s[0], 0, csm, off, pb, psum);
     if constexpr (SPLIT) {
       sp_s1 = s[1];
@@ -426,7 +469,7 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
       }
     }
   } else {
-    int cur = next_valid(0);
+    int cur = next_valid(e0 * NSUB);
     if (cur < total) issue(cur, buf0);
     while (cur < total) {
       wait_vm0();
@@ -446,6 +489,10 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
   }
 
   // ---- epilogue
+  if (PART) {
+    part_flush();
+    return;
+  }
   if (MASS) {
     mass_flush();
     __syncthreads();  // every wavefront's shares are in mslot
@@ -473,6 +520,88 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
       }
   }
   if (g == 0) a.lse_out[hT + R.row] = l_row > 0.f ? (m_run + log2f(l_row)) * kLn2 : -INFINITY;
+}
+
+// From the (maximum, sum) pairs of every list entry and row: the rows' LSE and
+// the block masses mass[kb] = Σ_rows sum·2^(max - M) / L, unlisted blocks 0.
+// One 512-thread workgroup per list row.  The pairs (8 bytes per entry and
+// row, ≤ kPartBytes per launch) were just written, so both readings of them
+// come mostly from the caches; the loads go four ahead.
+template <int BS>
+__global__ __launch_bounds__(512) void mass_merge_kernel(AttnArgs a) {
+  constexpr int NT = 512, NP = NT / BS, NR = BS / 64, NW = NT / 64;
+  __shared__ float pm[NP][BS], pl[NP][BS];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int64_t lrow = a.part_row0 + static_cast<int64_t>(blockIdx.x);
+  const int h = static_cast<int>(lrow / a.QB), qb = static_cast<int>(lrow % a.QB);
+  const int n = min(a.kv_num[lrow], a.maxkv);
+  const int32_t* lst = a.kv_idx + lrow * a.maxkv;
+  const float2* part = a.part + static_cast<int64_t>(blockIdx.x) * a.maxkv * BS;
+  float* mrow = a.mass + lrow * a.QB;
+  for (int i = tid; i < a.QB; i += NT) mrow[i] = 0.f;
+  {
+    // thread (row, part): the entries part, part + NP, ..; an entry after the
+    // q-block has no visible key and no pair
+    const int r = tid % BS, p = tid / BS;
+    float M = -INFINITY, L = 0.f;
+    for (int eb = p; eb < n; eb += 4 * NP) {
+      float2 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = eb + i * NP;
+        v[i] = e < n && lst[e] <= qb ? part[static_cast<int64_t>(e) * BS + r] : make_float2(-INFINITY, 0.f);
+      }
+      float m4 = M;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m4 = fmaxf(m4, v[i].x);
+      // -inf maxima come with a zero sum (or a NaN one, which stays)
+      L *= M == m4 ? 1.f : __builtin_amdgcn_exp2f(M - m4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) L += v[i].x == m4 ? v[i].y : v[i].y * __builtin_amdgcn_exp2f(v[i].x - m4);
+      M = m4;
+    }
+    pm[p][r] = M;
+    pl[p][r] = L;
+  }
+  __syncthreads();
+  float M[NR], inv[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int r = lane + 64 * i;
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) m = fmaxf(m, pm[p][r]);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) l += pm[p][r] == m ? pl[p][r] : pl[p][r] * __builtin_amdgcn_exp2f(pm[p][r] - m);
+    M[i] = m;
+    inv[i] = l > 0.f ? 1.f / l : 0.f;
+    if (wave == 0) a.lse_out[static_cast<int64_t>(h) * a.T + static_cast<int64_t>(qb) * BS + r] =
+        l > 0.f ? (m + log2f(l)) * kLn2 : -INFINITY;
+  }
+  // four entries' loads in flight per wavefront
+  constexpr int NE = 4;
+  for (int eb = wave * NE; eb < n; eb += NW * NE) {
+    float2 v[NE][NR];
+    int kb[NE];
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      kb[j] = eb + j < n ? lst[eb + j] : INT32_MAX;
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        v[j][i] = kb[j] <= qb ? part[static_cast<int64_t>(eb + j) * BS + lane + 64 * i] : make_float2(-INFINITY, 0.f);
+    }
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      float s = 0.f;
+      // a row without a sum (inv = 0) has no mass, but keeps a NaN
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        s += inv[i] > 0.f ? v[j][i].y * (__builtin_amdgcn_exp2f(v[j][i].x - M[i]) * inv[i]) : v[j][i].y * 0.f;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (lane == 0 && kb[j] <= qb) mrow[kb[j]] = s;
+    }
+  }
 }
 
 template <int BS, int KIND = kFwdAttn>
@@ -595,6 +724,93 @@ extern "C" int scope_attn_fwd(const scope_attn_params* p, const uint16_t* q, con
   else
     launch_fwd<128>(a, p->bias_mode, grid, s);
   return check_launch("attn_fwd_kernel");
+}
+
+namespace {
+// Scratch of the one-pass block mass: rows of at most this many bytes are in
+// flight at a time (it stays in the 256 MB last-level cache), more run as
+// further pairs of launches.
+constexpr int64_t kPartBytes = 256ll << 20;
+
+int64_t part_row_bytes(const scope_attn_params* p) { return static_cast<int64_t>(p->maxkv) * p->bs * 8; }
+int64_t part_rows(const scope_attn_params* p) {
+  const int64_t rows = static_cast<int64_t>(p->H) * (p->T / p->bs);
+  return std::max<int64_t>(1, std::min(rows, kPartBytes / part_row_bytes(p)));
+}
+}  // namespace
+
+extern "C" int64_t scope_attn_block_mass_workspace_bytes(const scope_attn_params* p) {
+  if (!p || p->maxkv < 1 || p->bs < 1 || p->T < p->bs || p->H < 1) return 0;
+  return part_rows(p) * part_row_bytes(p);
+}
+
+// One pass over the scores: the lists are cut into runs of entries, a
+// workgroup each, that write every row's (maximum, sum) per entry; a second
+// kernel forms the LSE and the masses of a row from them.  Against the
+// two-pass kernels (LSE, then masses) it forms the scores once, and a
+// q-block's list is no longer one workgroup's serial chain: at T = 16384, H = 4
+// the two passes took 291 + 330 us (their 512 workgroups are all resident from
+// the start, so the longest list is the time), this takes 220 + 22; the
+// teacher's call 629 -> 250 us there, 664 -> 118 at H = 1, 2456 -> 1560 at
+// T = 65536, H = 8.  What bounds it now is the scores' VALU work (about 170
+// instructions and 32 exponentials per 64-key tile and wavefront for 22 MFMAs).
+extern "C" int scope_attn_block_mass_ws(const scope_attn_params* p, const uint16_t* q, const uint16_t* k,
+                                        const int32_t* kv_num, const int32_t* kv_idx, const int32_t* docs,
+                                        const int32_t* ds_tok_end, const void* table, const float* coeff_cos,
+                                        const float* coeff_sin, const float* b0, const float* slope,
+                                        const float* delta_main, const float* width, float* lse, float* mass,
+                                        void* work, void* stream) {
+  int rc = validate_attn(p, q, k, k, kv_num, kv_idx, docs, ds_tok_end, table, coeff_cos, coeff_sin, b0, slope,
+                         delta_main, width, "scope_attn_block_mass_ws");
+  if (rc) return rc;
+  SCOPE_REQUIRE(lse && mass && work, "scope_attn_block_mass_ws: null output or workspace");
+  SCOPE_REQUIRE(p->T / p->bs <= 65536, "scope_attn_block_mass_ws: %lld key blocks (at most 65536)",
+                (long long)(p->T / p->bs));
+  AttnArgs a = make_args(p);
+  a.q = q;
+  a.k = k;
+  a.v = k;  // never staged
+  a.kv_num = kv_num;
+  a.kv_idx = kv_idx;
+  a.docs = docs;
+  a.ds_tok_end = ds_tok_end;
+  a.table = table;
+  a.coeff_cos = coeff_cos;
+  a.coeff_sin = coeff_sin;
+  a.b0 = b0;
+  a.slope = slope;
+  a.delta_main = delta_main;
+  a.width = width;
+  a.lse_out = lse;
+  a.mass = mass;
+  a.part = static_cast<float2*>(work);
+  const int64_t rows = static_cast<int64_t>(p->H) * a.QB, per = part_rows(p);
+  hipStream_t s = as_stream(stream);
+  for (int64_t r0 = 0; r0 < rows; r0 += per) {
+    a.part_row0 = static_cast<int>(r0);
+    a.part_rows = static_cast<int>(std::min(per, rows - r0));
+    // entries per workgroup: eight pay for its start (the Q rows and features)
+    // and still spread the lists (T = 16384, H = 4: 330 / 277 / 250 / 241 us a
+    // call with 2 / 4 / 8 / 16 entries; T = 65536, H = 8: 2411 / 1765 / 1563 /
+    // 1610 us); fewer where eight would leave some of the 768 resident
+    // workgroups (three per CU) without one
+    a.part_entries = static_cast<int>(
+        std::min<int64_t>(8, std::max<int64_t>(2, static_cast<int64_t>(a.part_rows) * a.maxkv / 768)));
+    const int64_t grid = static_cast<int64_t>(ceil_div(a.part_rows, 8)) * 8 * ceil_div(a.maxkv, a.part_entries);
+    if (p->bs == 256)
+      launch_fwd<256, kFwdPart>(a, p->bias_mode, static_cast<int>(grid), s);
+    else
+      launch_fwd<128, kFwdPart>(a, p->bias_mode, static_cast<int>(grid), s);
+    rc = check_launch("attn_fwd_kernel (entry sums)");
+    if (rc) return rc;
+    if (p->bs == 256)
+      hipLaunchKernelGGL(mass_merge_kernel<256>, dim3(a.part_rows), dim3(512), 0, s, a);
+    else
+      hipLaunchKernelGGL(mass_merge_kernel<128>, dim3(a.part_rows), dim3(512), 0, s, a);
+    rc = check_launch("mass_merge_kernel");
+    if (rc) return rc;
+  }
+  return SCOPE_OK;
 }
 
 extern "C" int scope_attn_block_mass(const scope_attn_params* p, const uint16_t* q, const uint16_t* k,

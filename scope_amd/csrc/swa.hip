@@ -171,9 +171,29 @@ __global__ __launch_bounds__(256) void swa_pad_kernel(int NB, const int32_t* __r
   if (j >= kv_num[qb]) kv_idx[i] = kv_idx[static_cast<int64_t>(qb) * w];
 }
 
+// dense document-causal lists: row (h, qb) = blocks first .. qb, the tail qb
+__global__ __launch_bounds__(256) void causal_lists_kernel(const int32_t* __restrict__ ds_local, int NB,
+                                                           int32_t* __restrict__ kv_num,
+                                                           int32_t* __restrict__ kv_idx) {
+  const int qb = blockIdx.x % NB;
+  const int first = ds_local[qb];
+  if (threadIdx.x == 0) kv_num[blockIdx.x] = qb - first + 1;
+  int32_t* row = kv_idx + static_cast<int64_t>(blockIdx.x) * NB;
+  for (int e = threadIdx.x; e < NB; e += 256) row[e] = min(first + e, qb);
+}
+
 }  // namespace scope
 
 using namespace scope;
+
+extern "C" int scope_causal_lists(const int32_t* ds_local, int H, int NB, int32_t* kv_num, int32_t* kv_idx,
+                                  void* stream) {
+  SCOPE_REQUIRE(ds_local && kv_num && kv_idx, "scope_causal_lists: null pointer");
+  SCOPE_REQUIRE(H >= 1 && NB >= 1 && NB <= 65536 && static_cast<int64_t>(H) * NB < (1ll << 31),
+                "scope_causal_lists: H=%d, NB=%d", H, NB);
+  hipLaunchKernelGGL(causal_lists_kernel, dim3(H * NB), dim3(256), 0, as_stream(stream), ds_local, NB, kv_num, kv_idx);
+  return check_launch("causal_lists_kernel");
+}
 
 extern "C" int scope_swa_blockmask(const int32_t* docs, int64_t T, int bs, int window_blocks, int32_t* counts,
                                    int32_t* partial_idx, int32_t* full_idx, int32_t* kv_num_long,

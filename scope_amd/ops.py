@@ -780,11 +780,25 @@ def attn_block_mass(q, k, kv_num, kv_idx, docs, ds_tok_end, *, bs: int, scale: f
     H, T = prm.H, prm.T
     NB = T // bs
     lse = torch.empty((1, H, T), dtype=torch.float32, device=dev)
-    mass = torch.zeros((H, NB, NB), dtype=torch.float32, device=dev)
-    call("scope_attn_block_mass", C.byref(prm), _p(q), _p(k), _p(_i32(kv_num)), _p(kv_idx3),
+    mass = torch.empty((H, NB, NB), dtype=torch.float32, device=dev)
+    ws = torch.empty(max(16, query("scope_attn_block_mass_workspace_bytes", C.byref(prm))), dtype=torch.uint8,
+                     device=dev)
+    call("scope_attn_block_mass_ws", C.byref(prm), _p(q), _p(k), _p(_i32(kv_num)), _p(kv_idx3),
          _p(_i32(docs.reshape(-1))), _p(_i32(ds_tok_end)), _p(table), _p(_f32(coeff_cos)), _p(_f32(coeff_sin)),
-         _p(_f32(b0)), _p(_f32(slope)), _p(_f32(delta_main)), _p(_f32(width)), _p(lse), _p(mass), _stream(dev))
+         _p(_f32(b0)), _p(_f32(slope)), _p(_f32(delta_main)), _p(_f32(width)), _p(lse), _p(mass), _p(ws), _stream(dev))
     return mass, lse
+
+
+def causal_lists(ds_local: torch.Tensor, H: int):
+    """The dense document-causal lists (kv_num [H,NB], kv_idx [H,NB,NB]): row
+    (h, qb) lists the blocks ds_local[qb] .. qb, its tail repeats qb."""
+    dev = _gpu("causal_lists", ds_local)
+    ds_local = _i32(ds_local.reshape(-1))
+    NB = ds_local.numel()
+    kv_num = torch.empty((H, NB), dtype=torch.int32, device=dev)
+    kv_idx = torch.empty((H, NB, NB), dtype=torch.int32, device=dev)
+    call("scope_causal_lists", _p(ds_local), int(H), NB, _p(kv_num), _p(kv_idx), _stream(dev))
+    return kv_num, kv_idx
 
 
 def decode_attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, kv_num: torch.Tensor,

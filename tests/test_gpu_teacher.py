@@ -1,5 +1,5 @@
 """Teacher block mass (scoped_medium.py:1799-1819) on the GPU
-(scope_attn_block_mass) against the fp64 oracle: the teacher's dense
+(scope_attn_block_mass_ws) against the fp64 oracle: the teacher's dense
 document-causal attention with the token-offset band term and slope, a
 pointer list with the block-offset bias, and the row-sum invariant at the
 training shape.  Bar (written in each comparison): |got - ref| <= 2e-2 +
@@ -94,3 +94,54 @@ def test_teacher_mass_row_sums_at_training_shape():
             want = res[(0, qb)][0].sum(0)
             ok, worst = tol_check(got[h, qb].cpu(), want)
             assert ok, f"head {h} q-block {qb}: worst tolerance ratio {worst:.3f}"
+
+
+@pytest.mark.parametrize("bs,T,H,mode", [(128, 128, 1, "token"), (128, 2176, 3, "token"), (256, 1280, 2, "block"),
+                                         (256, 256, 1, "none"), (128, 4096, 1, "gate")])
+def test_block_mass_one_pass_against_two_passes(bs, T, H, mode):
+    """The one-pass masses and LSE (scope_attn_block_mass_ws) against the
+    two-pass entry point on the same lists: one block, odd block counts, an
+    empty row, ragged lists.  Both are fp32 sums of the same probabilities
+    (exp2 to 1 ulp, at most bs·2^11 terms added in another order): masses of
+    at most bs differ by less than bs·2^-18, the LSE by 2^-18·(1 + |lse|)."""
+    import ctypes as C
+
+    from scope_amd import _lib, ops
+    from scope_amd.attention import spectral_table
+
+    print(f"block mass one/two passes bs={bs} T={T} H={H} {mode}", flush=True)
+    NB = T // bs
+    docs = docs_with_boundaries(T, min(3, NB), seed=51)
+    kv_num, kv_idx = random_blockscore_mask(H, T, bs, docs, window=2, n_global=1, budget=3, seed=52)
+    if NB > 2:
+        kv_num[0, 1] = 0
+    q, k, _ = qkv(H, T, seed=53)
+    A, B = band_coefficients(q)
+    bias = {"gate": "token"}.get(mode, mode)
+    kw = dict(bs=bs, scale=SCALE, beta=BETA, bias_mode=bias)
+    if bias != "none":
+        kw.update(table=spectral_table(omegas_block(8).to(DEV), T, bs, bias), coeff_cos=A.to(DEV), coeff_sin=B.to(DEV))
+    dm = wd = None
+    if mode == "gate":
+        g = torch.Generator().manual_seed(54)
+        dm, wd = (torch.rand((1, H, T), generator=g) * s for s in (1024.0, 256.0))
+        kw.update(delta_main=dm.to(DEV), width=wd.to(DEV), gate_kind="softplus", ramp_lambda=0.2, tau=64.0)
+    ds_end = torch.from_numpy(doc_start_blocks(docs.numpy(), bs)[2])
+    dev = [t.to(DEV).contiguous() for t in (q, k, kv_num, kv_idx, docs, ds_end)]
+    mass, lse = ops.attn_block_mass(*dev, **kw)
+    qd, kd, num, idx, dd, de = dev
+    prm = ops._attn_params(qd, kd, kd, qd, bs=bs, maxkv=idx.shape[-1], scale=SCALE, beta=BETA,
+                           bias_mode=ops.BIAS_MODES[bias], K=0 if bias == "none" else 8, use_slope=False,
+                           subtract_b0=False, gate_kind=int(mode == "gate"), ramp_lambda=0.2, tau=64.0)
+    m2 = torch.zeros_like(mass)
+    l2 = torch.empty_like(lse)
+    p = lambda t: None if t is None else C.c_void_p(t.data_ptr())  # noqa: E731
+    opt = [kw.get(n) for n in ("table", "coeff_cos", "coeff_sin", "b0", "slope", "delta_main", "width")]
+    _lib.call("scope_attn_block_mass", C.byref(prm), p(qd), p(kd), p(num), p(idx), p(dd), p(de), *(p(t) for t in opt),
+              p(l2), p(m2), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isinf(lse), torch.isinf(l2))
+    fin = torch.isfinite(l2)
+    assert ((lse - l2).abs()[fin] <= 2.0 ** -18 * (1 + l2.abs()[fin])).all()
+    assert (mass - m2).abs().max().item() <= bs * 2.0 ** -18
+    assert torch.equal(mass > 0, m2 > 0)
