@@ -584,6 +584,50 @@ int scope_decoder_step_prologue(const int64_t* tok, const int64_t* t_dev, int64_
                                 const uint16_t* ve0, const uint16_t* ve1, const uint16_t* ve2, uint16_t* x0,
                                 uint16_t* ve_out, void* stream);
 
+/* One decoder token through every layer (the position *t_dev = t, inside a
+ * q-block: the lists of layer.kv_num / kv_idx are those of t's block): what
+ * scope_decoder_step_prologue, then per layer scope_decoder_gemv (qkv),
+ * scope_decode_attn_glue_at and scope_decoder_gemv (projection, MLP) compute,
+ * in one launch of resident workgroups.  tokens[t], docs[t] and cache rows t
+ * are written, x_out [dm] gets the last layer's output, *t_dev becomes t + 1.
+ * The layers' lambdas are (1, 0), the U-net skips' weights 1.
+ *   layers      device array of p->layers records (qkv NULL: no attention;
+ *               ve: value-embedding table 0..2, -1 none); kv_num [H],
+ *               kv_idx [H][maxkv]
+ *   work        scope_decoder_step_workspace_bytes bytes, zeroed once, then
+ *               owned by this decoder (word 1: status, 1 after a wait of more
+ *               than spin_ticks (100 MHz); the step then gives NaN)
+ *   host_status pinned host int that also gets the status, or NULL
+ * scope_decoder_step_supported: whether the shape is served and the current
+ * device holds all workgroups at once. */
+typedef struct {
+  const uint16_t* qkv;      /* [3·H·D][dm] */
+  const uint16_t* proj;     /* [dm][H·D] */
+  const uint16_t* mlp_fc;   /* [mlp][dm] */
+  const uint16_t* mlp_proj; /* [dm][mlp] */
+  uint16_t* k_cache;
+  uint16_t* v_cache;
+  const int32_t* kv_num;
+  const int32_t* kv_idx;
+  float va, vb;
+  int ve;
+  int reserved;
+} scope_decoder_layer;
+
+typedef struct {
+  int layers, H, D, dm, mlp, bs, maxkv;
+  float scale, eps;
+  int64_t T_cap, vocab, eot, rot_rows, rot_st, k_sh, k_st, v_sh, v_st;
+  uint64_t spin_ticks;
+} scope_decoder_step_params;
+
+int scope_decoder_step_supported(const scope_decoder_step_params* p);
+int64_t scope_decoder_step_workspace_bytes(const scope_decoder_step_params* p);
+int scope_decoder_step(const scope_decoder_step_params* p, const scope_decoder_layer* layers, const int64_t* tok,
+                       int64_t* t_dev, int64_t* tokens, int32_t* docs, const uint16_t* embed, const uint16_t* ve0,
+                       const uint16_t* ve1, const uint16_t* ve2, const float* cos_t, const float* sin_t,
+                       uint16_t* x_out, void* work, int32_t* host_status, void* stream);
+
 /* The greedy choice of the decoder's token loop: *out = the index of the
  * largest of x[0..n) fp32 (the first on ties, as torch.argmax; NaN values
  * are never chosen; all NaN gives 0).  One workgroup.  No counterpart in the

@@ -80,6 +80,19 @@ class DecodeParams(C.Structure):
                 ("v_st", c_int64), ("o_sh", c_int64)]
 
 
+class DecoderLayer(C.Structure):
+    _fields_ = [("qkv", c_void_p), ("proj", c_void_p), ("mlp_fc", c_void_p), ("mlp_proj", c_void_p),
+                ("k_cache", c_void_p), ("v_cache", c_void_p), ("kv_num", c_void_p), ("kv_idx", c_void_p),
+                ("va", c_float), ("vb", c_float), ("ve", c_int), ("reserved", c_int)]
+
+
+class DecoderStepParams(C.Structure):
+    _fields_ = [("layers", c_int), ("H", c_int), ("D", c_int), ("dm", c_int), ("mlp", c_int), ("bs", c_int),
+                ("maxkv", c_int), ("scale", c_float), ("eps", c_float), ("T_cap", c_int64), ("vocab", c_int64),
+                ("eot", c_int64), ("rot_rows", c_int64), ("rot_st", c_int64), ("k_sh", c_int64), ("k_st", c_int64),
+                ("v_sh", c_int64), ("v_st", c_int64), ("spin_ticks", c_uint64)]
+
+
 P = c_void_p
 _PROTOS = {
     "scope_abi_version": (c_int, []),
@@ -126,6 +139,9 @@ _PROTOS = {
     "scope_decoder_qkv_glue": (c_int, [c_int, c_int, c_int, c_int64, c_float, c_float, c_float, P, P, P, P, P,
                                        c_int64, c_int64, P, P, P, c_int64, c_int64, c_int64, c_int64, c_int, P]),
     "scope_decoder_gemv": (c_int, [c_int, c_int, c_int64, c_int, c_float, c_int, P, P, P, P, P, P, P]),
+    "scope_decoder_step_supported": (c_int, [C.POINTER(DecoderStepParams)]),
+    "scope_decoder_step_workspace_bytes": (c_int64, [C.POINTER(DecoderStepParams)]),
+    "scope_decoder_step": (c_int, [C.POINTER(DecoderStepParams)] + [P] * 15),
     "scope_argmax_f32": (c_int, [P, c_int64, P, P]),
     "scope_decode_attn_glue_at": (c_int, [C.POINTER(DecodeParams), P, P, P, c_float, c_float, c_float, P, P, c_int64,
                                           c_int64, P, P, P, P, P, P, P, P, P, P]),

@@ -19,6 +19,9 @@ make greedy decoding trivial).
   new token's query, the only one known), and keeps it for the block's other
   positions; the attention of the token runs ``scope_decode_attn`` over the
   list.  When t closes a block, its key mean joins the candidates.
+* At the default width a step that opens no block runs every layer in one
+  launch (``ops.decoder_step``); other configurations take a chain of fused
+  kernels per layer.
 * The steps inside a block (neither opening nor closing it) run as one
   captured HIP graph (``torch.cuda.CUDAGraph``), replayed per token: the
   position lives on the device (``_t_dev``; cache and document writes index
@@ -147,6 +150,11 @@ class ScopeDecoder(nn.Module):
         self._g_tok = None
         self._g_out = None
         self._g_warm = 0
+        # the one-launch step (``_fused``): the table of the layers' tensors, the
+        # addresses it was made from, and the status its waits set (pinned)
+        self._step_key: tuple | None = None
+        self._step_table = None
+        self._step_status = None
 
     # ---- pieces shared by prefill and step -------------------------------------
     def _ve(self, tok: torch.Tensor):
@@ -227,6 +235,43 @@ class ScopeDecoder(nn.Module):
         return self._logits(x) if all_logits else self._logits(x[-1:])[0]
 
     # ---- one decode step ---------------------------------------------------------
+    def _fused(self):
+        """The arguments of ``ops.decoder_step`` (table of the layers' current
+        tensors, workspace), or None when a step has to run layer by layer:
+        other sizes than the library serves, mixing weights other than the
+        model's initial ones, or a device too small for it."""
+        cfg, n = self.cfg, len(self.skip_weights)
+        if self.device.type != "cuda" or any(w != 1.0 for w in self.skip_weights) \
+                or any(lay["lambdas"] != (1.0, 0.0) for lay in self.layers) or len(self.layers) != 2 * n:
+            return None
+        names = ("qkv", "proj", "mlp_fc", "mlp_proj")
+        key = tuple(lay[m].data_ptr() if m in lay else 0 for lay in self.layers for m in names) \
+            + tuple(lay.get("vlam", ()) for lay in self.layers) \
+            + tuple(0 if t is None else t.data_ptr() for ts in (self.k_cache, self.v_cache, self.list_num, self.list_idx)
+                    for t in ts)
+        if key != self._step_key:
+            ve = [0, 1, 2] + [-1] * (cfg.num_layers - 6) + [0, 1, 2]
+            layers = []
+            for i, lay in enumerate(self.layers):
+                va, vb = lay.get("vlam", (0.0, 0.0))
+                layers.append(dict(qkv=lay.get("qkv"), proj=lay.get("proj"), mlp_fc=lay["mlp_fc"],
+                                   mlp_proj=lay["mlp_proj"], k_cache=self.k_cache[i], v_cache=self.v_cache[i],
+                                   kv_num=self.list_num[i], kv_idx=self.list_idx[i], ve=ve[i], va=va, vb=vb))
+            cache = next((c for c in self.k_cache if c is not None), None)
+            self._step_table = None
+            if cache is not None and cfg.num_layers >= 6:
+                self._step_table = ops.decoder_step_table(layers, dict(
+                    layers=cfg.num_layers, H=cfg.num_heads, D=cfg.head_dim, dm=cfg.model_dim, mlp=4 * cfg.model_dim,
+                    bs=cfg.block_size, maxkv=cfg.window + cfg.budget + cfg.n_global, scale=cfg.attn_scale,
+                    eps=torch.finfo(torch.float32).eps, T_cap=self.max_len, vocab=cfg.vocab_size, eot=EOT,
+                    rot_rows=self.rotary.cos.shape[0], rot_st=self.rotary.cos.stride(0), k_sh=cache.stride(0),
+                    k_st=cache.stride(1), v_sh=cache.stride(0), v_st=cache.stride(1),
+                    spin_ticks=20 * 100_000_000), cache.device)
+            if self._step_status is None:
+                self._step_status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            self._step_key = key
+        return self._step_table
+
     def _body(self, tok: torch.Tensor, t: int, opens: bool, closes: bool) -> torch.Tensor:
         """The step at the position held in ``_t_dev`` (= t), then _t_dev += 1.
         ``opens`` / ``closes`` (eager steps only) add the block's reselection /
@@ -234,6 +279,15 @@ class ScopeDecoder(nn.Module):
         cfg = self.cfg
         bs = cfg.block_size
         td = self._t_dev
+        fused = None if opens else self._fused()
+        if fused is not None:
+            x = ops.decoder_step(*fused, tok, td, self.tokens, self.docs, self.embed, self.value_embeds,
+                                 self.rotary.cos, self.rotary.sin, self._step_status)
+            if closes:  # the block is complete: its key means join the candidates
+                for kbar, kc in zip(self.kbar, self.k_cache):
+                    if kbar is not None:
+                        kbar[:, t // bs] = kc[:, t // bs * bs:t + 1].float().mean(dim=1)
+            return ops.decoder_gemv(x, self.lm_head, norm=True, epi="logit")
         # token and document bookkeeping, the embedding, its norm and the
         # value embeddings in one kernel
         x0, ve3 = ops.decoder_step_prologue(tok, td, self.tokens, self.docs, self.embed, self.value_embeds, eot=EOT)
@@ -311,6 +365,8 @@ class ScopeDecoder(nn.Module):
         t = self.t
         if t >= self.max_len:
             raise ValueError("step: the cache is full")
+        if self._step_status is not None and int(self._step_status[0]):
+            raise RuntimeError("step: an earlier step's workgroups waited too long for each other; its logits are NaN")
         if not isinstance(token, torch.Tensor) or not token.is_cuda:  # a host token is checked here
             if not 0 <= int(token) < self.cfg.vocab_size:
                 raise ValueError(f"step: token {int(token)} outside the vocabulary [0, {self.cfg.vocab_size})")
@@ -338,6 +394,7 @@ class ScopeDecoder(nn.Module):
             return out
         if self._graph is None:
             self._g_tok = tok.clone()
+            self._g_table = self._fused()  # made outside the capture, alive as long as the graph
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):
                 self._g_out = self._body(self._g_tok, -1, False, False)

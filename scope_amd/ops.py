@@ -1007,6 +1007,63 @@ def decoder_step_prologue(tok: torch.Tensor, t_dev: torch.Tensor, tokens: torch.
     return x0, ve
 
 
+def decoder_step_table(layers, params: dict, device: torch.device):
+    """(params struct, device table of the layer records, workspace) of
+    ``decoder_step``, or None when the library's one-launch step does not
+    serve the decoder (its sizes, or a device that cannot hold the kernel's
+    workgroups at once).  ``layers``: dicts with qkv / proj (None without
+    attention), mlp_fc, mlp_proj, k_cache, v_cache, kv_num, kv_idx, ve, va, vb."""
+    prm = _lib.DecoderStepParams(**params)
+    with torch.cuda.device(device):
+        if not query("scope_decoder_step_supported", C.byref(prm)):
+            return None
+    hd, dm, mlp = prm.H * prm.D, prm.dm, prm.mlp
+    shapes = dict(qkv=(3 * hd, dm), proj=(dm, hd), mlp_fc=(mlp, dm), mlp_proj=(dm, mlp))
+    rec = (_lib.DecoderLayer * len(layers))()
+    for r, lay in zip(rec, layers):
+        for n_, shape in shapes.items():
+            w = lay[n_]
+            if w is None and n_ in ("qkv", "proj"):
+                continue
+            if w.dtype != torch.bfloat16 or tuple(w.shape) != shape or not w.is_contiguous() or w.data_ptr() % 16 \
+                    or w.device != device:
+                return None
+            setattr(r, n_, w.data_ptr())
+        if lay["qkv"] is not None:
+            for n_ in ("k_cache", "v_cache", "kv_num", "kv_idx"):
+                setattr(r, n_, lay[n_].data_ptr())
+        r.ve, r.va, r.vb = lay["ve"], lay["va"], lay["vb"]
+    table = torch.frombuffer(bytearray(bytes(rec)), dtype=torch.uint8).to(device)
+    work = torch.zeros(int(query("scope_decoder_step_workspace_bytes", C.byref(prm))), dtype=torch.uint8, device=device)
+    return prm, table, work
+
+
+def decoder_step(prm, table: torch.Tensor, work: torch.Tensor, tok: torch.Tensor, t_dev: torch.Tensor,
+                 tokens: torch.Tensor, docs: torch.Tensor, embed: torch.Tensor, value_embeds, cos: torch.Tensor,
+                 sin: torch.Tensor, host_status: torch.Tensor | None = None) -> torch.Tensor:
+    """One decoder token through every layer in one launch
+    (``scope_decoder_step``) -> the last layer's output [dm] bf16.  prm, table
+    and work come from ``decoder_step_table``; the tensors behind the table
+    must be alive until the step has run."""
+    dev = _gpu("decoder_step", table, work, tok, t_dev, tokens, docs, embed, cos, sin, *value_embeds)
+    if tok.dtype != torch.int64 or tok.numel() != 1 or t_dev.dtype != torch.int64 or t_dev.numel() != 1:
+        raise RuntimeError("decoder_step: tok and t_dev must be one int64 element each")
+    if tokens.dtype != torch.int64 or docs.dtype != torch.int32 or tokens.numel() != prm.T_cap \
+            or docs.numel() != prm.T_cap or not tokens.is_contiguous() or not docs.is_contiguous():
+        raise RuntimeError("decoder_step: tokens int64 [T_cap] and docs int32 [T_cap], contiguous")
+    for tb in (embed, *value_embeds):
+        if tb.dtype != torch.bfloat16 or not tb.is_contiguous() or tb.shape != (prm.vocab, prm.dm):
+            raise RuntimeError(f"decoder_step: embedding tables must be contiguous bfloat16 [{prm.vocab}, {prm.dm}]")
+    if cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != (prm.rot_rows, prm.D // 2) \
+            or cos.stride() != (prm.rot_st, 1) or sin.stride() != cos.stride() or sin.shape != cos.shape:
+        raise RuntimeError("decoder_step: cos/sin must be float32 [rot_rows, D/2]")
+    x = torch.empty(prm.dm, dtype=torch.bfloat16, device=dev)
+    tabs = list(value_embeds) + [None] * (3 - len(value_embeds))
+    call("scope_decoder_step", C.byref(prm), _p(table), _p(tok), _p(t_dev), _p(tokens), _p(docs), _p(embed),
+         *(_p(v) for v in tabs), _p(cos), _p(sin), _p(x), _p(work), _p(host_status), _stream(dev))
+    return x
+
+
 def attn_bwd(q, k, v, out, dout, lse, kv_num, kv_idx, q_off, q_list, docs, ds_tok_end, *, bs: int, scale: float,
              beta: float = 0.5, bias_mode: str = "none", table=None, coeff_cos=None, coeff_sin=None, b0=None,
              slope=None, delta_main=None, width=None, use_slope=False, subtract_b0=False, gate_kind="none",

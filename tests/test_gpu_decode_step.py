@@ -1,0 +1,116 @@
+"""The decoder's one-launch token step (scope_decoder_step) against the
+layer-by-layer step on the same state.  Both round the same bf16 values at the
+same places and differ in the order of their fp32 sums only, so single bf16
+results may round to a neighbour and travel on: the bar on logits (of scale
+15 ± 0.5) is the one of the token loop against the prefill, 5e-2, and on the
+caches 2^-4 (a few bf16 steps of values of order 1 to 4)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _model(max_len, fused=True, layers=16, window=4, budget=4, **kw):
+    from scope_amd.decode import DecoderConfig, ScopeDecoder
+
+    m = ScopeDecoder(DecoderConfig(num_layers=layers, window=window, budget=budget), max_len=max_len, device=DEV, seed=5,
+                     **kw)
+    if not fused:
+        m._fused = lambda: None
+    return m
+
+
+def _close(a, b, t):
+    err = max((x[:, :t].float() - y[:, :t].float()).abs().max().item() for x, y in zip(a.k_cache + a.v_cache,
+              b.k_cache + b.v_cache) if x is not None)
+    assert err <= 2.0 ** -4, f"cache difference {err:.3e}"
+    err = max((x - y).abs().max().item() for x, y in zip(a.kbar, b.kbar) if x is not None)
+    assert err <= 2.0 ** -4, f"key-mean difference {err:.3e}"
+
+
+@pytest.mark.parametrize("layers,window,budget,T0,n", [(16, 4, 4, 256, 133), (8, 2, 1, 128, 9), (6, 20, 11, 1152, 5)])
+def test_step_equals_layer_by_layer(layers, window, budget, T0, n):
+    """A block opening, its steps (a document opens inside), its closing and
+    the next opening; the smallest and the widest lists (4 and 32 entries)."""
+    print(f"one-launch step: {layers} layers, lists of {window + budget + 1}, {n} steps", flush=True)
+    g = torch.Generator().manual_seed(9)
+    toks = torch.randint(0, 50256, (T0 + n,), generator=g)
+    toks[[T0 // 2, T0 + 4]] = 50256
+    one, ref = (_model(T0 + 256, f, layers, window, budget, use_graph=False) for f in (True, False))
+    assert one._fused() is not None
+    for m in (one, ref):
+        m.prefill(toks[:T0])
+    worst = 0.0
+    for s in range(n):
+        a, b = one.step(toks[T0 + s]), ref.step(toks[T0 + s])
+        worst = max(worst, (a - b).abs().max().item())
+        assert worst <= 5e-2, f"step {s}: {worst:.3e}"
+    assert torch.equal(one.docs, ref.docs) and torch.equal(one.tokens, ref.tokens)
+    assert int(one._t_dev) == int(ref._t_dev) == T0 + n
+    _close(one, ref, T0 + n)
+    print(f"  max logit difference {worst:.3e}", flush=True)
+
+
+def test_token_outside_the_vocabulary_and_other_sizes():
+    """A device token outside the vocabulary leaves tokens and docs as they
+    are and enters as a zero row, as in the layer-by-layer step; other widths
+    are not served."""
+    one, ref = (_model(256, f, 6, use_graph=False) for f in (True, False))
+    toks = torch.randint(0, 50256, (130,), generator=torch.Generator().manual_seed(1))
+    bad = torch.tensor([60000], device=DEV)
+    for m in (one, ref):
+        m.prefill(toks[:128])
+        m.step(toks[128])
+    a, b = one.step(bad), ref.step(bad)
+    assert (a - b).abs().max().item() <= 5e-2
+    assert torch.equal(one.docs, ref.docs) and torch.equal(one.tokens, ref.tokens)
+    from scope_amd.decode import DecoderConfig, ScopeDecoder
+
+    small = ScopeDecoder(DecoderConfig(num_layers=6, num_heads=2, model_dim=256), max_len=256, device=DEV, seed=1)
+    assert small._fused() is None
+
+
+def test_two_decoders_on_two_streams():
+    """Steps of two decoders queued on two streams at the same time (each
+    needs all of its workgroups resident) give what they give one by one."""
+    toks = torch.randint(0, 50256, (160,), generator=torch.Generator().manual_seed(2)).to(DEV)
+    ms = [_model(256, True, 6, use_graph=False) for _ in range(2)]
+    want = []
+    for rnd in range(2):
+        outs = [[], []]
+        for m in ms:
+            m.prefill(toks[:128])
+            m.step(toks[128:129])
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()] if rnd else [torch.cuda.current_stream()] * 2
+        for s in range(129, 155):
+            for i, m in enumerate(ms):
+                with torch.cuda.stream(streams[i]):
+                    outs[i].append(m.step(toks[s:s + 1]))
+        torch.cuda.synchronize()
+        if rnd == 0:
+            want = outs
+    for i in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(outs[i], want[i])), f"decoder {i}"
+
+
+def test_expired_wait_gives_nan_and_raises():
+    """With the status word set (as a wait that lasted too long leaves it) the
+    kernel ends at once with NaN rows; with the host's copy set, step raises."""
+    m = _model(256, True, 6, use_graph=False)
+    toks = torch.randint(0, 50256, (140,), generator=torch.Generator().manual_seed(3))
+    m.prefill(toks[:128])
+    m.step(toks[128])
+    work = m._fused()[2]
+    work[4:8].copy_(torch.tensor([1, 0, 0, 0], dtype=torch.uint8, device=DEV))
+    assert bool(torch.isnan(m.step(toks[129])).all())
+    work[4:8].zero_()
+    m.prefill(toks[:128])
+    m.step(toks[128])
+    assert bool(torch.isfinite(m.step(toks[129])).all())
+    m._step_status[0] = 1
+    with pytest.raises(RuntimeError, match="waited too long"):
+        m.step(toks[130])
