@@ -584,6 +584,15 @@ int scope_decoder_step_prologue(const int64_t* tok, const int64_t* t_dev, int64_
                                 const uint16_t* ve0, const uint16_t* ve1, const uint16_t* ve2, uint16_t* x0,
                                 uint16_t* ve_out, void* stream);
 
+/* The prefill's steps between its matrix products.
+ * relu2: h [n] bf16 := bf16(relu(h)^2) in place (scoped_medium.py:491).
+ * add_norm: s = bf16(x + y); then bf16(s + skip) with skip, bf16(s + s) with
+ * skip_self, or s, to x_out; xn = its RMS norm
+ * (scoped_medium.py:266-267, :507-510, :607).  Rows of dm <= 4096. */
+int scope_decoder_relu2(uint16_t* h, int64_t n, void* stream);
+int scope_decoder_add_norm(int64_t T, int dm, float eps, const uint16_t* x, const uint16_t* y, const uint16_t* skip,
+                           int skip_self, uint16_t* x_out, uint16_t* xn, void* stream);
+
 /* One decoder token through every layer (the position *t_dev = t, inside a
  * q-block: the lists of layer.kv_num / kv_idx are those of t's block): what
  * scope_decoder_step_prologue, then per layer scope_decoder_gemv (qkv),

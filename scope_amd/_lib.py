@@ -139,6 +139,8 @@ _PROTOS = {
     "scope_decoder_qkv_glue": (c_int, [c_int, c_int, c_int, c_int64, c_float, c_float, c_float, P, P, P, P, P,
                                        c_int64, c_int64, P, P, P, c_int64, c_int64, c_int64, c_int64, c_int, P]),
     "scope_decoder_gemv": (c_int, [c_int, c_int, c_int64, c_int, c_float, c_int, P, P, P, P, P, P, P]),
+    "scope_decoder_relu2": (c_int, [P, c_int64, P]),
+    "scope_decoder_add_norm": (c_int, [c_int64, c_int, c_float, P, P, P, c_int, P, P, P]),
     "scope_decoder_step_supported": (c_int, [C.POINTER(DecoderStepParams)]),
     "scope_decoder_step_workspace_bytes": (c_int64, [C.POINTER(DecoderStepParams)]),
     "scope_decoder_step": (c_int, [C.POINTER(DecoderStepParams)] + [P] * 15),

@@ -271,68 +271,194 @@ __global__ __launch_bounds__(kDecD) void decode_merge_kernel(scope_decode_params
 // result to bf16), v = a·v + b·ve (each product and the sum rounded to bf16,
 // as bf16 tensor arithmetic does; b·ve dropped without ve).  q goes to
 // q_out [T, H, D]; k and v go to row pos[t] of the caches (cache_at_pos) or
-// to row t.  One 128-thread workgroup per (token, head).
-__global__ __launch_bounds__(kDecD) void qkv_glue_kernel(int H, int64_t rows, float eps, float va, float vb,
-                                                          const uint16_t* __restrict__ qkv,
-                                                          const uint16_t* __restrict__ ve,
-                                                          const int64_t* __restrict__ pos,
-                                                          const float* __restrict__ cos_t,
-                                                          const float* __restrict__ sin_t, int64_t rot_rows,
-                                                          int64_t rot_st, uint16_t* __restrict__ q_out,
-                                                          uint16_t* __restrict__ kc, uint16_t* __restrict__ vc,
-                                                          int64_t k_sh, int64_t k_st, int64_t v_sh, int64_t v_st,
-                                                          int cache_at_pos) {
-  constexpr int D = kDecD, HD = kDecD / 2;
-  const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-  const int64_t p = pos[t];
-  const int64_t w = cache_at_pos ? p : t;  // the k/v row written
-  uint16_t* qo = q_out + (static_cast<int64_t>(t) * H + h) * D + d;
-  if (p < 0 || p >= rot_rows || w < 0 || w >= rows) {  // uniform over the workgroup: no rotary row / no cache row
-    *qo = 0;
-    return;
-  }
-  const uint16_t* row = qkv + static_cast<int64_t>(t) * 3 * H * D;
-  const float q = bf16_to_f32(row[h * D + d]);
-  const float k = bf16_to_f32(row[(H + h) * D + d]);
-  const float v = bf16_to_f32(row[(2 * H + h) * D + d]);
-  __shared__ float part[2][2];
-  __shared__ float xs[2][D];
-  float sq = q * q, sk = k * k;
-  for (int o = 32; o > 0; o >>= 1) {
-    sq += __shfl_xor(sq, o, kWave);
-    sk += __shfl_xor(sk, o, kWave);
-  }
-  if ((d & 63) == 0) {
-    part[d >> 6][0] = sq;
-    part[d >> 6][1] = sk;
-  }
-  __syncthreads();
-  const float rq = 1.f / sqrtf((part[0][0] + part[1][0]) / D + eps);
-  const float rk = 1.f / sqrtf((part[0][1] + part[1][1]) / D + eps);
-  const float qn = bf16_to_f32(f32_to_bf16(__fmul_rn(q, rq)));
-  const float kn = bf16_to_f32(f32_to_bf16(__fmul_rn(k, rk)));
-  xs[0][d] = qn;
-  xs[1][d] = kn;
-  __syncthreads();
-  const float c = cos_t[p * rot_st + (d % HD)], sn = sin_t[p * rot_st + (d % HD)];
-  float yq, yk;
-  if (d < HD) {
-    yq = __fadd_rn(__fmul_rn(qn, c), __fmul_rn(xs[0][d + HD], sn));
-    yk = __fadd_rn(__fmul_rn(kn, c), __fmul_rn(xs[1][d + HD], sn));
-  } else {
-    yq = __fadd_rn(__fmul_rn(xs[0][d - HD], -sn), __fmul_rn(qn, c));
-    yk = __fadd_rn(__fmul_rn(xs[1][d - HD], -sn), __fmul_rn(kn, c));
-  }
-  *qo = f32_to_bf16(yq);
-  kc[h * k_sh + w * k_st + d] = f32_to_bf16(yk);
-  float vv = bf16_to_f32(f32_to_bf16(__fmul_rn(va, v)));
-  if (ve) {
-    const float e = bf16_to_f32(ve[static_cast<int64_t>(t) * H * D + h * D + d]);
-    vv = bf16_to_f32(f32_to_bf16(__fadd_rn(vv, bf16_to_f32(f32_to_bf16(__fmul_rn(vb, e))))));
-  }
-  vc[h * v_sh + w * v_st + d] = f32_to_bf16(vv);
+// to row t.
+//
+// Bound by memory: 16 lanes per (token, head), 8 features (one 16-byte chunk
+// of q, k, v, ve and of each output) per lane, the rotation's partner feature
+// d ± 64 in lane l ^ 8.  T = 32768, H = 8: 85 us, 5.5 TB/s of its 0.47 GB
+// (230 us with a 128-thread workgroup per row and 2-byte accesses).  The sums
+// of squares add in the order of that kernel (and of the one-token kernels'
+// wavefront sums), so the bf16 results are the same bit for bit.
+template <int XOR>
+__device__ __forceinline__ float lane_xor(float x) {
+  if constexpr (XOR == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));
+  if constexpr (XOR == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, true));
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), (XOR << 10) | 0x1f));
 }
 
+// Σ x² over the 128 features of a 16-lane group, added as a wavefront's xor
+// tree over features (32, 16, 8, 4, 2, 1) and then the two halves
+__device__ __forceinline__ float sum_sq128(const float (&x)[8]) {
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    s[i] = x[i] * x[i];
+    s[i] += lane_xor<4>(s[i]);
+    s[i] += lane_xor<2>(s[i]);
+    s[i] += lane_xor<1>(s[i]);
+  }
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+    for (int i = 0; i < o; ++i) s[i] += s[i + o];
+  return s[0] + lane_xor<8>(s[0]);
+}
+
+__device__ __forceinline__ void unpack8(const uint4& u, float (&f)[8]) {
+  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = __uint_as_float(w[i] << 16);
+    f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
+  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
+}
+__device__ __forceinline__ float round_bf16(float x) { return bf16_to_f32(f32_to_bf16(x)); }
+
+// bf16 of the rotated bf16(x·r) (r = 1/rms): lanes 0-7 of the group hold
+// features below 64, lanes 8-15 their partners
+__device__ __forceinline__ uint4 norm_rotate8(const float (&x)[8], float eps, const float (&c)[8], const float (&sn)[8],
+                                              bool low) {
+  const float r = 1.f / sqrtf(sum_sq128(x) / kDecD + eps);
+  float y[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float xn = round_bf16(__fmul_rn(x[i], r)), o = lane_xor<8>(xn);
+    y[i] = low ? __fadd_rn(__fmul_rn(xn, c[i]), __fmul_rn(o, sn[i])) : __fadd_rn(__fmul_rn(o, -sn[i]), __fmul_rn(xn, c[i]));
+  }
+  return pack8(y);
+}
+
+// eight bf16 values at p: one chunk, or (A = false: rows that are not 16-byte
+// aligned) one by one
+template <bool A>
+__device__ __forceinline__ void load8(const uint16_t* p, float (&f)[8]) {
+  if constexpr (A) {
+    unpack8(*reinterpret_cast<const uint4*>(p), f);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = bf16_to_f32(p[i]);
+  }
+}
+template <bool A>
+__device__ __forceinline__ void store8(uint16_t* p, const uint4& u) {
+  if constexpr (A) {
+    *reinterpret_cast<uint4*>(p) = u;
+  } else {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[2 * i] = static_cast<uint16_t>(w[i]), p[2 * i + 1] = static_cast<uint16_t>(w[i] >> 16);
+  }
+}
+
+template <bool A>
+__global__ __launch_bounds__(256) void qkv_glue_kernel(int64_t pairs, int H, int64_t rows, float eps, float va, float vb,
+                                                       const uint16_t* __restrict__ qkv,
+                                                       const uint16_t* __restrict__ ve,
+                                                       const int64_t* __restrict__ pos,
+                                                       const float* __restrict__ cos_t,
+                                                       const float* __restrict__ sin_t, int64_t rot_rows,
+                                                       int64_t rot_st, uint16_t* __restrict__ q_out,
+                                                       uint16_t* __restrict__ kc, uint16_t* __restrict__ vc,
+                                                       int64_t k_sh, int64_t k_st, int64_t v_sh, int64_t v_st,
+                                                       int cache_at_pos) {
+  constexpr int D = kDecD, HD = kDecD / 2;
+  const int64_t pair = static_cast<int64_t>(blockIdx.x) * 16 + threadIdx.x / 16;  // (token, head), head fastest
+  if (pair >= pairs) return;  // whole groups of 16 lanes leave together
+  const int ch = threadIdx.x % 16;
+  const int64_t t = pair / H;
+  const int h = static_cast<int>(pair % H);
+  const int64_t p = pos[t];
+  const int64_t w = cache_at_pos ? p : t;  // the k/v row written
+  uint16_t* qo = q_out + pair * D + 8 * ch;
+  if (p < 0 || p >= rot_rows || w < 0 || w >= rows) {  // the same in the group: no rotary row / no cache row
+    store8<A>(qo, make_uint4(0, 0, 0, 0));
+    return;
+  }
+  const uint16_t* row = qkv + t * 3 * H * D + h * D + 8 * ch;
+  float q[8], k[8], v[8], c[8], sn[8];
+  load8<A>(row, q);
+  load8<A>(row + H * D, k);
+  load8<A>(row + 2 * H * D, v);
+  const int d0 = 8 * ch % HD;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) c[i] = cos_t[p * rot_st + d0 + i], sn[i] = sin_t[p * rot_st + d0 + i];
+  store8<A>(qo, norm_rotate8(q, eps, c, sn, ch < 8));
+  store8<A>(kc + h * k_sh + w * k_st + 8 * ch, norm_rotate8(k, eps, c, sn, ch < 8));
+  float e[8];
+  if (ve) load8<A>(ve + pair * D + 8 * ch, e);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    v[i] = round_bf16(__fmul_rn(va, v[i]));
+    if (ve) v[i] = __fadd_rn(v[i], round_bf16(__fmul_rn(vb, e[i])));
+  }
+  store8<A>(vc + h * v_sh + w * v_st + 8 * ch, pack8(v));
+}
+
+// The prefill's steps between its matrix products, each one pass:
+// h := bf16(relu(h)²) in place, eight values per thread (T = 32768 rows of
+// 4096: 83 us, 6.5 TB/s; relu and square apart took 168).
+__global__ __launch_bounds__(256) void relu2_kernel(uint4* __restrict__ h, int64_t n8) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n8) return;
+  float f[8];
+  unpack8(h[i], f);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float r = f[j] < 0.f ? 0.f : f[j];  // keeps a NaN, as relu does
+    f[j] = __fmul_rn(r, r);
+  }
+  h[i] = pack8(f);
+}
+
+// s = bf16(x + y), then with skip bf16(s + skip) (skip_self: bf16(s + s)), to x_out; xn = F.rms_norm of it (48 us for 32768 rows of 1024, 5.6 TB/s;
+// the add and the norm apart took 31 + 34).  A wavefront per
+// row of dm, KC = ceil(dm / 512) chunks of 8 per lane.
+template <int KC>
+__global__ __launch_bounds__(256) void add_norm_kernel(int64_t T, int dm, float eps, const uint16_t* __restrict__ x,
+                                                       const uint16_t* __restrict__ y, const uint16_t* __restrict__ skip,
+                                                       int skip_self, uint16_t* __restrict__ x_out,
+                                                       uint16_t* __restrict__ xn) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / 64;
+  if (t >= T) return;  // wavefront-uniform
+  const int lane = threadIdx.x % 64;
+  float s[KC][8], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < KC; ++c) {
+    const int ch = lane + 64 * c;
+    const bool in = 8 * ch < dm;
+    const int64_t at = t * dm + 8 * ch;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[c][i] = 0.f;
+    if (!in) continue;
+    float b[8];
+    unpack8(*reinterpret_cast<const uint4*>(x + at), s[c]);
+    unpack8(*reinterpret_cast<const uint4*>(y + at), b);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[c][i] = round_bf16(__fadd_rn(s[c][i], b[i]));
+    if (skip || skip_self) {
+      if (skip) unpack8(*reinterpret_cast<const uint4*>(skip + at), b);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[c][i] = round_bf16(__fadd_rn(s[c][i], skip ? b[i] : s[c][i]));
+    }
+    *reinterpret_cast<uint4*>(x_out + at) = pack8(s[c]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss = fmaf(s[c][i], s[c][i], ss);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+  const float r = 1.f / sqrtf(ss / dm + eps);
+#pragma unroll
+  for (int c = 0; c < KC; ++c) {
+    const int ch = lane + 64 * c;
+    if (8 * ch >= dm) continue;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[c][i] = __fmul_rn(s[c][i], r);
+    *reinterpret_cast<uint4*>(xn + t * dm + 8 * ch) = pack8(s[c]);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Row-vector products of the decoder's token step, fused with the ops around
@@ -351,15 +477,6 @@ __global__ __launch_bounds__(kDecD) void qkv_glue_kernel(int H, int64_t rows, fl
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 4;
 enum { kGemvPlain = 0, kGemvRelu2 = 1, kGemvResid = 2, kGemvLogit = 3 };
-
-__device__ __forceinline__ void unpack8(const uint4& u, float (&f)[8]) {
-  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = __uint_as_float(w[i] << 16);
-    f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-  }
-}
 
 template <int K, int EPI, int R>
 __global__ __launch_bounds__(64 * kGemvWaves) void gemv_kernel(int N, int64_t ldw, int norm, float eps,
@@ -646,9 +763,47 @@ extern "C" int scope_decoder_qkv_glue(int T, int H, int D, int64_t rows, float e
   SCOPE_REQUIRE(D == kDecD, "scope_decoder_qkv_glue: head dim D=%d (supported: 128)", D);
   SCOPE_REQUIRE(T >= 1 && T <= 2147483647 && H >= 1 && H <= 65535 && rows >= 1 && rot_rows >= 1 && rot_st >= D / 2,
                 "scope_decoder_qkv_glue: bad T=%d / H=%d / rows=%lld / rotary table", T, H, (long long)rows);
-  hipLaunchKernelGGL(qkv_glue_kernel, dim3(T, H), dim3(kDecD), 0, as_stream(stream), H, rows, eps, va, vb, qkv, ve,
-                     pos, cos_t, sin_t, rot_rows, rot_st, q_out, k_out, v_out, k_sh, k_st, v_sh, v_st, cache_at_pos);
+  const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  const bool al = a16(qkv) && (!ve || a16(ve)) && a16(q_out) && a16(k_out) && a16(v_out) && k_sh % 8 == 0 &&
+                  k_st % 8 == 0 && v_sh % 8 == 0 && v_st % 8 == 0;
+  const int64_t pairs = static_cast<int64_t>(T) * H;
+  SCOPE_REQUIRE(pairs <= (1ll << 34), "scope_decoder_qkv_glue: T=%d, H=%d", T, H);
+  const dim3 grid(static_cast<unsigned>((pairs + 15) / 16)), blk(256);
+  hipStream_t st = as_stream(stream);
+  if (al)
+    hipLaunchKernelGGL(qkv_glue_kernel<true>, grid, blk, 0, st, pairs, H, rows, eps, va, vb, qkv, ve, pos, cos_t, sin_t,
+                       rot_rows, rot_st, q_out, k_out, v_out, k_sh, k_st, v_sh, v_st, cache_at_pos);
+  else
+    hipLaunchKernelGGL(qkv_glue_kernel<false>, grid, blk, 0, st, pairs, H, rows, eps, va, vb, qkv, ve, pos, cos_t, sin_t,
+                       rot_rows, rot_st, q_out, k_out, v_out, k_sh, k_st, v_sh, v_st, cache_at_pos);
   return check_launch("qkv_glue_kernel");
+}
+
+extern "C" int scope_decoder_relu2(uint16_t* h, int64_t n, void* stream) {
+  SCOPE_REQUIRE(h && n >= 8 && n % 8 == 0 && n <= (1ll << 40) && (reinterpret_cast<uintptr_t>(h) & 15) == 0,
+                "scope_decoder_relu2: n=%lld must be a positive multiple of 8, h 16-byte aligned", (long long)n);
+  hipLaunchKernelGGL(relu2_kernel, dim3(static_cast<unsigned>((n / 8 + 255) / 256)), dim3(256), 0, as_stream(stream),
+                     reinterpret_cast<uint4*>(h), n / 8);
+  return check_launch("relu2_kernel");
+}
+
+extern "C" int scope_decoder_add_norm(int64_t T, int dm, float eps, const uint16_t* x, const uint16_t* y,
+                                      const uint16_t* skip, int skip_self, uint16_t* x_out, uint16_t* xn,
+                                      void* stream) {
+  SCOPE_REQUIRE(x && y && x_out && xn, "scope_decoder_add_norm: null pointer");
+  SCOPE_REQUIRE(T >= 1 && T < (1ll << 32) && dm >= 8 && dm % 8 == 0 && dm <= 4096,
+                "scope_decoder_add_norm: T=%lld rows of dm=%d (a multiple of 8, at most 4096)", (long long)T, dm);
+  SCOPE_REQUIRE(!(skip && skip_self), "scope_decoder_add_norm: skip and skip_self");
+  const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  SCOPE_REQUIRE(a16(x) && a16(y) && (!skip || a16(skip)) && a16(x_out) && a16(xn),
+                "scope_decoder_add_norm: tensors must be 16-byte aligned");
+  const dim3 grid(static_cast<unsigned>((T + 3) / 4)), blk(256);
+  hipStream_t s = as_stream(stream);
+  if (dm <= 512) hipLaunchKernelGGL(add_norm_kernel<1>, grid, blk, 0, s, T, dm, eps, x, y, skip, skip_self, x_out, xn);
+  else if (dm <= 1024) hipLaunchKernelGGL(add_norm_kernel<2>, grid, blk, 0, s, T, dm, eps, x, y, skip, skip_self, x_out, xn);
+  else if (dm <= 2048) hipLaunchKernelGGL(add_norm_kernel<4>, grid, blk, 0, s, T, dm, eps, x, y, skip, skip_self, x_out, xn);
+  else hipLaunchKernelGGL(add_norm_kernel<8>, grid, blk, 0, s, T, dm, eps, x, y, skip, skip_self, x_out, xn);
+  return check_launch("add_norm_kernel");
 }
 
 template <int K, int R>

@@ -175,18 +175,15 @@ class ScopeDecoder(nn.Module):
         return ops.decoder_qkv_glue(qkv, ve, pos, self.rotary.cos, self.rotary.sin, heads=cfg.num_heads, va=a,
                                     vb=b if ve is not None else 0.0, k_out=kc, v_out=vc)
 
-    def _mlp(self, lay, x: torch.Tensor) -> torch.Tensor:
-        h = F.linear(_norm(x), lay["mlp_fc"])
-        return F.linear(F.relu(h).square(), lay["mlp_proj"])
-
     def _logits(self, x: torch.Tensor) -> torch.Tensor:
         return 30 * torch.sigmoid(F.linear(_norm(x), self.lm_head).float() / 7.5)
 
-    def _select(self, qbar: torch.Tensor, kbar: torch.Tensor, nb: int, return_logits: bool = False):
-        """Block-scoring lists of blocks 0..nb-1 from q̄, k̄ [H, nb, D]."""
+    def _select(self, qbar: torch.Tensor, kbar: torch.Tensor, nb: int, return_logits: bool = False, ds=None):
+        """Block-scoring lists of blocks 0..nb-1 from q̄, k̄ [H, nb, D]; ``ds``:
+        their document starts, when the caller has them."""
         cfg = self.cfg
         T = nb * cfg.block_size
-        ds_ptr, ds_local, _ = ops.doc_starts(self.docs[:T], cfg.block_size)
+        ds_ptr, ds_local, _ = ds or ops.doc_starts(self.docs[:T], cfg.block_size)
         return ops.pointer_select(ds_ptr, ds_local, bs=cfg.block_size, NB=nb, H=cfg.num_heads, window=cfg.window,
                                   n_global=cfg.n_global, budget=cfg.budget, qbar=qbar, kbar=kbar, temp=1.0,
                                   logit_scale=cfg.block_size / math.sqrt(cfg.head_dim), noise="none",
@@ -206,29 +203,51 @@ class ScopeDecoder(nn.Module):
         self.tokens[:T] = tok
         self.docs[:T] = (tok == EOT).cumsum(0).to(torch.int32)
         docs = self.docs[:T]
-        _, _, ds_tok_end = ops.doc_starts(docs, bs)
+        ds = ops.doc_starts(docs, bs)
         pos = torch.arange(T, device=self.device)
         ve = self._ve(tok)
         x = x0 = _norm(F.embedding(tok, self.embed))
-        skips = []
-        n = len(self.skip_weights)
+        skips: list = []
+        n, L = len(self.skip_weights), len(self.layers)
+        # with the model's initial mixing weights the residual adds, the U-net
+        # skips and the norms between the products run as one pass each
+        plain = all(w == 1.0 for w in self.skip_weights) and L == 2 * n and cfg.model_dim % 8 == 0 \
+            and cfg.model_dim <= 4096 and all(lay["lambdas"] == (1.0, 0.0) for lay in self.layers)
+        xn = _norm(x)
         for i, lay in enumerate(self.layers):
-            if i >= n:
-                x = _skip(x, self.skip_weights[i - n], skips.pop())
-            a, b = lay["lambdas"]
-            x = _mix(a, b, x, x0)
+            if not plain:
+                if i >= n:
+                    x = _skip(x, self.skip_weights[i - n], skips.pop())
+                a, b = lay["lambdas"]
+                x = _mix(a, b, x, x0)
+                xn = _norm(x)
             if "qkv" in lay:
-                q, kc, vc = self._qkv(lay, _norm(x), ve[i], pos, i)  # k, v into cache rows 0 .. T-1
+                q, kc, vc = self._qkv(lay, xn, ve[i], pos, i)  # k, v into cache rows 0 .. T-1
                 qh, kh, vh = q.transpose(0, 1), kc[:, :T], vc[:, :T]  # [H, T, D] views
                 qbar, kbar = ops.block_means(qh, kh, bs)
                 self.kbar[i][:, :T // bs] = kbar
-                kv_num, kv_idx, _ = self._select(qbar, kbar, T // bs)
-                y, _ = ops.attn_fwd(qh[None], kh[None], vh[None], kv_num, kv_idx, docs, ds_tok_end, bs=bs,
+                kv_num, kv_idx, _ = self._select(qbar, kbar, T // bs, ds=ds)
+                y, _ = ops.attn_fwd(qh[None], kh[None], vh[None], kv_num, kv_idx, docs, ds[2], bs=bs,
                                     scale=cfg.attn_scale, check=False)
-                x = x + F.linear(y[0].transpose(0, 1).reshape(T, -1), lay["proj"])
-            x = x + self._mlp(lay, x)
-            if i < n:
-                skips.append(x)
+                y = F.linear(y[0].transpose(0, 1).reshape(T, -1), lay["proj"])
+                if plain:
+                    x, xn = ops.decoder_add_norm(x, y)
+                else:
+                    x = x + y
+                    xn = _norm(x)
+            y = F.linear(ops.decoder_relu2(F.linear(xn, lay["mlp_fc"])), lay["mlp_proj"])
+            if not plain:
+                x = x + y
+                if i < n:
+                    skips.append(x)
+            elif i == L - 1:
+                x = x + y
+            elif i == n - 1:  # layer n takes this layer's own output as its skip
+                x, xn = ops.decoder_add_norm(x, y, skip_self=True)
+            else:
+                x, xn = ops.decoder_add_norm(x, y, skip=skips.pop() if i >= n else None)
+                if i < n:
+                    skips.append(x)
         self.t = T
         self._t_dev.fill_(T)
         self.have_lists = False

@@ -965,6 +965,32 @@ def decoder_gemv(x: torch.Tensor, w: torch.Tensor, *, norm: bool = False, epi: s
     return (out, xout) if addx is not None else out
 
 
+def decoder_relu2(h: torch.Tensor) -> torch.Tensor:
+    """relu(h)² in place (bf16, contiguous, a multiple of 8 elements), rounded
+    as ``F.relu(h).square()`` rounds it."""
+    dev = _gpu("decoder_relu2", h)
+    if h.dtype != torch.bfloat16 or not h.is_contiguous():
+        raise RuntimeError("decoder_relu2: h must be a contiguous bfloat16 tensor")
+    call("scope_decoder_relu2", _p(h), h.numel(), _stream(dev))
+    return h
+
+
+def decoder_add_norm(x: torch.Tensor, y: torch.Tensor, *, skip: torch.Tensor | None = None, skip_self: bool = False,
+                     eps: float | None = None):
+    """(x', F.rms_norm(x')) with s = x + y and x' = s, s + skip, or s + s with
+    ``skip_self``; each sum rounded to bf16.  x, y, skip [T, dm] bf16
+    contiguous, dm a multiple of 8 up to 4096."""
+    dev = _gpu("decoder_add_norm", x, y, skip)
+    for n_, t in (("x", x), ("y", y), ("skip", skip)):
+        if t is not None and (t.dtype != torch.bfloat16 or t.dim() != 2 or not t.is_contiguous() or t.shape != x.shape):
+            raise RuntimeError(f"decoder_add_norm: {n_} must be a contiguous bfloat16 [T, dm]")
+    T, dm = x.shape
+    out, xn = torch.empty_like(x), torch.empty_like(x)
+    e = torch.finfo(torch.float32).eps if eps is None else float(eps)
+    call("scope_decoder_add_norm", T, dm, e, _p(x), _p(y), _p(skip), int(bool(skip_self)), _p(out), _p(xn), _stream(dev))
+    return out, xn
+
+
 def argmax(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """Index of the largest element of a contiguous fp32 vector (the first on
     ties, as torch.argmax; NaN never chosen), as an int64 [1] tensor on the
