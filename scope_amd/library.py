@@ -1,7 +1,8 @@
 """The C ABI registered as torch operators: ``torch.ops.scope.*``.
 
-Each operator is a ``torch.library.custom_op`` whose implementation calls the
-gfx950 library through ``scope_amd.ops`` (device pointers, the current
+Each operator (``_Operator``, a direct registration with torch's dispatcher)
+has an implementation that calls the gfx950 library through
+``scope_amd.ops`` (device pointers, the current
 stream); a ``register_fake`` shape function lets it trace under FakeTensor,
 ``torch.compile`` (fullgraph) and AOT autograd without a graph break, and the
 differentiable ones carry ``register_autograd`` backward formulas.  This is
@@ -51,6 +52,78 @@ _I32, _F32 = torch.int32, torch.float32
 _HEAD_NAMES = ("coeff_cos", "coeff_sin", "slope", "b0", "delta_star", "pi", "budget_logits", "delta_main", "width")
 
 
+_LIB = torch.library.Library(_NS, "FRAGMENT")
+
+
+class _Operator:
+    """``scope::name`` defined and registered with the dispatcher directly.
+
+    An operator made by ``torch.library.custom_op`` has the same schema,
+    kernels and autograd behaviour, but its Python wrappers run on every
+    call: 25 us for a small operator, 150 us for one with the 26 arguments of
+    the attention and an autograd formula (the arguments' defaults are looked
+    up one by one, and there are none here).  A training layer's dozen
+    operators were bound by that below T = 8192 or so: a step of T = 2048
+    took 579 us forward and backward, now 270."""
+
+    def __init__(self, name, fn):
+        self._name = name
+        schema = torch.library.infer_schema(fn, mutates_args=())
+        _LIB.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
+        _LIB.impl(name, torch._disable_dynamo(fn), "CompositeExplicitAutograd")
+        self._op = getattr(getattr(torch.ops, _NS), name).default
+        self._setup = self._backward = self._function = None
+        _LIB.impl(name, self._autograd, "Autograd")
+        self.__doc__ = fn.__doc__
+
+    def __call__(self, *args, **kwargs):
+        return self._op(*args, **kwargs)
+
+    def register_fake(self, fn):
+        torch.library.register_fake(f"{_NS}::{self._name}", fn, lib=_LIB)
+        return fn
+
+    def register_autograd(self, backward, *, setup_context):
+        """``setup_context(ctx, inputs, output)`` and ``backward(ctx, *grads)``
+        as in ``torch.library.register_autograd``."""
+        self._backward, self._setup = backward, setup_context
+
+    def _make_function(self):
+        op, name, setup, formula = self._op, self._name, self._setup, self._backward
+
+        def forward(ctx, *args):
+            args = args if formula is not None else args[0]
+            with torch._C._AutoDispatchBelowAutograd():
+                out = op(*args)
+            if setup is not None:
+                setup(ctx, args, out)
+            return out
+
+        def backward(ctx, *grads):
+            if formula is None:
+                raise RuntimeError(f"Trying to backward through {_NS}::{name} but no autograd formula was registered.")
+            return formula(ctx, *grads)
+
+        return type(f"Scope_{name}", (torch.autograd.Function,),
+                    dict(forward=staticmethod(forward), backward=staticmethod(backward)))
+
+    def _autograd(self, *args):
+        if torch.is_grad_enabled():
+            tensors = [a for a in args if isinstance(a, Tensor)]
+            tensors += [b for a in args if isinstance(a, (list, tuple)) for b in a if isinstance(b, Tensor)]
+            if any(t.requires_grad for t in tensors):
+                if self._function is None:
+                    self._function = self._make_function()
+                # without a formula the tensors (a list's among them) only mark the outputs as not differentiable
+                return self._function.apply(*args) if self._backward is not None else self._function.apply(args, *tensors)
+        with torch._C._AutoDispatchBelowAutograd():
+            return self._op(*args)
+
+
+def _operator(name):
+    return lambda fn: _Operator(name, fn)
+
+
 def _none(dev: torch.device) -> Tensor:
     """The empty stand-in of an absent optional output."""
     return torch.empty(0, dtype=_F32, device=dev)
@@ -69,7 +142,7 @@ def seed_to_signed(seed: int) -> int:
 
 # ---------------------------------------------------------------------------
 # document starts
-@torch.library.custom_op(f"{_NS}::doc_starts", mutates_args=())
+@_operator("doc_starts")
 def doc_starts(docs: Tensor, bs: int, doc_clamp: bool, reset_len: int) -> tuple[Tensor, Tensor, Tensor]:
     return ops.doc_starts(docs, bs, doc_clamp=doc_clamp, reset_len=reset_len)
 
@@ -91,7 +164,7 @@ def ref_maxkv(T: int, bs: int, M: int, local_blocks: int, ptr_half_blocks: int, 
     return local + npk + min(max(global_blocks_cfg, 0), NB)
 
 
-@torch.library.custom_op(f"{_NS}::pointer_mask_ref", mutates_args=())
+@_operator("pointer_mask_ref")
 def pointer_mask_ref(delta_star: Tensor, budget_logits: Tensor, ds_ptr: Tensor, ds_local: Tensor,
                      gumbel_u: Optional[Tensor], bs: int, local_blocks: int, ptr_half_blocks: int,
                      global_blocks_cfg: int, global_active: int, radius_pi: bool, budget_rem: int, budget_temp: float,
@@ -118,7 +191,7 @@ def _(delta_star, budget_logits, ds_ptr, ds_local, gumbel_u, bs, local_blocks, p
 
 # ---------------------------------------------------------------------------
 # block-scoring selection
-@torch.library.custom_op(f"{_NS}::block_means", mutates_args=())
+@_operator("block_means")
 def block_means(q: Tensor, k: Tensor, bs: int) -> tuple[Tensor, Tensor]:
     return ops.block_means(q, k, bs)
 
@@ -129,7 +202,7 @@ def _(q, k, bs):
     return q.new_empty((H, T // bs, D), dtype=_F32), q.new_empty((H, T // bs, D), dtype=_F32)
 
 
-@torch.library.custom_op(f"{_NS}::block_means_docs", mutates_args=())
+@_operator("block_means_docs")
 def block_means_docs(q: Tensor, k: Tensor, docs: Tensor, bs: int, doc_clamp: bool,
                      reset_len: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     return ops.block_means_docs(q, k, docs, bs, doc_clamp=doc_clamp, reset_len=reset_len)
@@ -143,7 +216,7 @@ def _(q, k, docs, bs, doc_clamp, reset_len):
     return means + tuple(docs.new_empty(NB, dtype=_I32) for _ in range(3))
 
 
-@torch.library.custom_op(f"{_NS}::pointer_select", mutates_args=())
+@_operator("pointer_select")
 def pointer_select(ds_ptr: Tensor, ds_local: Tensor, qbar: Optional[Tensor], kbar: Optional[Tensor],
                    logits_in: Optional[Tensor], prior: Optional[Tensor], gumbel_u: Optional[Tensor], bs: int, NB: int,
                    H: int, window: int, n_global: int, budget: int, temp: float, logit_scale: float, noise_mode: int,
@@ -170,7 +243,7 @@ def _(ds_ptr, ds_local, qbar, kbar, logits_in, prior, gumbel_u, bs, NB, H, windo
 # ---------------------------------------------------------------------------
 # soft pointer weights (no reference counterpart: the reference selects under
 # torch.no_grad, model/attn_bias.py:623)
-@torch.library.custom_op(f"{_NS}::soft_pointer_bias", mutates_args=())
+@_operator("soft_pointer_bias")
 def soft_pointer_bias(q: Tensor, k: Tensor, kv_num: Tensor, kv_idx: Tensor, picks: Tensor, prior: Optional[Tensor],
                       bs: int, window: int, n_global: int, logit_scale: float,
                       soft_temp: float) -> tuple[Tensor, Tensor, Tensor]:
@@ -189,7 +262,7 @@ def _(q, k, kv_num, kv_idx, picks, prior, bs, window, n_global, logit_scale, sof
             q.new_empty((H, T // bs, D), dtype=_F32))
 
 
-@torch.library.custom_op(f"{_NS}::pair_bias_from_logits", mutates_args=())
+@_operator("pair_bias_from_logits")
 def pair_bias_from_logits(kv_num: Tensor, kv_idx: Tensor, picks: Tensor, logits: Tensor, bs: int, window: int,
                           n_global: int, soft_temp: float) -> Tensor:
     """The soft weights of the picks from given logits [H,QB,NB] (constants:
@@ -203,7 +276,7 @@ def _(kv_num, kv_idx, picks, logits, bs, window, n_global, soft_temp):
     return kv_idx.new_empty(kv_idx.shape, dtype=_F32)
 
 
-@torch.library.custom_op(f"{_NS}::soft_pointer_bwd", mutates_args=())
+@_operator("soft_pointer_bwd")
 def soft_pointer_bwd(qbar: Tensor, kbar: Tensor, kv_num: Tensor, kv_idx: Tensor, q_off: Tensor, q_list: Tensor,
                      pair_bias: Tensor, dpair_bias: Tensor, q_like: Tensor, k_like: Tensor, bs: int,
                      logit_scale: float, soft_temp: float) -> tuple[Tensor, Tensor]:
@@ -245,7 +318,7 @@ soft_pointer_bias.register_autograd(_soft_backward, setup_context=_soft_setup)
 
 # ---------------------------------------------------------------------------
 # transposed lists
-@torch.library.custom_op(f"{_NS}::transpose_blocks", mutates_args=())
+@_operator("transpose_blocks")
 def transpose_blocks(kv_num: Tensor, kv_idx: Tensor, NB: int) -> tuple[Tensor, Tensor]:
     """(q_off [H, NB+1], q_list [H, QB*MAXKV]); a head's entries past
     q_off[h, NB] are -1."""
@@ -260,7 +333,7 @@ def _(kv_num, kv_idx, NB):
 
 # ---------------------------------------------------------------------------
 # statistics
-@torch.library.custom_op(f"{_NS}::mask_stats", mutates_args=())
+@_operator("mask_stats")
 def mask_stats(delta_star: Optional[Tensor], pi: Optional[Tensor], ds_ptr_fwd: Optional[Tensor],
                ds_local_fwd: Optional[Tensor], kv_num: Optional[Tensor], radius: Optional[Tensor],
                picks: Optional[Tensor], ds_ptr: Optional[Tensor], ds_local: Optional[Tensor], H: int, QB: int,
@@ -290,7 +363,7 @@ def table_bytes(mode: int, T: int, bs: int) -> int:
     return (T // bs) * 16 * 4 if mode == 1 else (T * 32 * 2 if mode == 2 else 0)
 
 
-@torch.library.custom_op(f"{_NS}::spectral_table", mutates_args=())
+@_operator("spectral_table")
 def spectral_table(omegas: Tensor, T: int, bs: int, mode: int) -> Tensor:
     return ops.spectral_table(omegas, T, bs, {1: "block", 2: "token"}[mode])
 
@@ -306,7 +379,7 @@ _GATES = ("none", "softplus", "relu")
 _MODES = ("none", "block", "token")
 
 
-@torch.library.custom_op(f"{_NS}::attn_fwd", mutates_args=())
+@_operator("attn_fwd")
 def attn_fwd(q: Tensor, k: Tensor, v: Tensor, kv_num: Tensor, kv_idx: Tensor, docs: Tensor, ds_tok_end: Tensor,
              q_off: Tensor, q_list: Tensor, table: Optional[Tensor], coeff_cos: Optional[Tensor],
              coeff_sin: Optional[Tensor], b0: Optional[Tensor], slope: Optional[Tensor], delta_main: Optional[Tensor],
@@ -343,7 +416,7 @@ def bwd_outputs_present(bias_mode: int, K: int, need_coeff_grads: bool, use_slop
 _BWD_NAMES = ("dcoeff_cos", "dcoeff_sin", "db0", "dslope", "ddelta_main", "dwidth", "dpair_bias")
 
 
-@torch.library.custom_op(f"{_NS}::attn_bwd", mutates_args=())
+@_operator("attn_bwd")
 def attn_bwd(q: Tensor, k: Tensor, v: Tensor, out: Tensor, dout: Tensor, lse: Tensor, kv_num: Tensor,
              kv_idx: Tensor, q_off: Tensor, q_list: Tensor, docs: Tensor, ds_tok_end: Tensor, table: Optional[Tensor],
              coeff_cos: Optional[Tensor], coeff_sin: Optional[Tensor], b0: Optional[Tensor], slope: Optional[Tensor],
@@ -434,7 +507,7 @@ def _unpack(iprm: Sequence[int], fprm: Sequence[float]) -> dict:
     return d
 
 
-@torch.library.custom_op(f"{_NS}::coeff_head_fwd", mutates_args=())
+@_operator("coeff_head_fwd")
 def coeff_head_fwd(y: Tensor, omegas: Tensor, log_omegas: Tensor, cos_mean: Optional[Tensor],
                    sin_mean: Optional[Tensor], iprm: list[int],
                    fprm: list[float]) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor,
@@ -454,7 +527,7 @@ def _(y, omegas, log_omegas, cos_mean, sin_mean, iprm, fprm):
     return tuple(e(shp[n], dtype=_F32) for n in _HEAD_NAMES) + (e(6, dtype=_F32),)
 
 
-@torch.library.custom_op(f"{_NS}::coeff_head_bwd", mutates_args=())
+@_operator("coeff_head_bwd")
 def coeff_head_bwd(y: Tensor, omegas: Tensor, log_omegas: Tensor, cos_mean: Optional[Tensor],
                    sin_mean: Optional[Tensor], grads: list[Optional[Tensor]], g_reg: Optional[Tensor], reg: Tensor,
                    iprm: list[int], fprm: list[float]) -> Tensor:
@@ -490,7 +563,7 @@ coeff_head_fwd.register_autograd(_head_backward, setup_context=_head_setup)
 # ---------------------------------------------------------------------------
 # The head's MLP (model/attn_bias.py:271-276, applied at :380-398)
 # ---------------------------------------------------------------------------
-@torch.library.custom_op(f"{_NS}::linear_wgrad", mutates_args=())
+@_operator("linear_wgrad")
 def linear_wgrad(a: Tensor, b: Tensor, round_bf16: bool) -> tuple[Tensor, Tensor]:
     """dw [M, N] = Σ_r a[r]^T b[r], db [M] = Σ_r a[r] over the bf16 rows of
     a [..., M] and b [..., N] (fp32, rounded to bf16 with ``round_bf16``)."""
@@ -502,7 +575,7 @@ def _(a, b, round_bf16):
     return a.new_empty((a.shape[-1], b.shape[-1]), dtype=_F32), a.new_empty(a.shape[-1], dtype=_F32)
 
 
-@torch.library.custom_op(f"{_NS}::coeff_mlp_bwd", mutates_args=())
+@_operator("coeff_mlp_bwd")
 def coeff_mlp_bwd(q: Tensor, gy: Tensor, w1: Tensor, b1: Tensor, w2: Tensor,
                   b2: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """The row-wise backward of the fused MLP: (dq, dz1, x1, gy padded to 64
@@ -517,7 +590,7 @@ def _(q, gy, w1, b1, w2, b2):
             q.new_empty(lead + (64,)))
 
 
-@torch.library.custom_op(f"{_NS}::coeff_mlp_bwd_wgrad", mutates_args=())
+@_operator("coeff_mlp_bwd_wgrad")
 def coeff_mlp_bwd_wgrad(q: Tensor, gy: Tensor, w1: Tensor, b1: Tensor, w2: Tensor,
                         b2: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     """The whole MLP backward on the fused kernels: (dq bf16, dw1, db1, dw2,
@@ -535,7 +608,7 @@ def _(q, gy, w1, b1, w2, b2):
             f((O, w2.shape[1])), f((O,)))
 
 
-@torch.library.custom_op(f"{_NS}::coeff_mlp", mutates_args=())
+@_operator("coeff_mlp")
 def coeff_mlp(q: Tensor, w1: Tensor, b1: Tensor, w2: Tensor, b2: Tensor) -> Tensor:
     """The head's shared MLP on q [..., D]: y = Linear(w2, b2)(SiLU(Linear(w1,
     b1)(q))) with the weights cast to q's dtype (model/attn_bias.py:380-386).

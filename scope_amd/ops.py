@@ -60,7 +60,8 @@ def call(name: str, *args) -> None:
 
 
 def _stream(dev: torch.device):
-    return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    # the raw handle of torch.cuda.current_stream(dev), without building its Python object
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(dev.index))
 
 
 def _gpu(name: str, *ts: torch.Tensor | None) -> torch.device:
