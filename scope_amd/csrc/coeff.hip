@@ -105,10 +105,63 @@ __device__ __forceinline__ void coeff_peak(const scope_coeff_params& p, const vo
   R.th = p.use_slope ? tanhf(load_y(y, bf, base + 5 * M)) : 0.f;
 }
 
-// e_mk for one peak (the caller normalises)
-__device__ __forceinline__ float coeff_e(const float* logw, int k, float mu, float sg) {
-  const float d = logw[k] - mu;
-  return expf(-(d * d) / (2.f * (sg * sg)));
+// The M·K exponentials and sine-cosine pairs of a row are the head's work
+// (about 0.4 TB/s of its bytes with the library's forms), so the three
+// functions here leave out what their arguments never need.  Errors against
+// fp64 over 4 M arguments, library's in brackets: sin and cos 1.7e-8 rms (1.8e-8),
+// 7.0e-8 at most (7.2e-8); exp2 of a reduced argument is the library's own form.
+//
+// sin and cos of |x| < kSincosMax: x - n·π/2 in two steps (n·1.57079637 fits
+// 41 bits and cancels exactly in the fma), Taylor polynomials on [-π/4, π/4]
+// to x^9 and x^10 (remainders 2e-9 and 1e-10), the quadrant by n mod 4.
+constexpr float kSincosMax = 65536.f;
+__device__ __forceinline__ void sincos_reduced(float x, float& s, float& c) {
+  const float n = rintf(x * 0.636619772f);
+  const float r = fmaf(n, 4.37113883e-8f, fmaf(-n, 1.57079637f, x));
+  const float z = r * r;
+  float p = fmaf(z, 2.75573192e-6f, -1.98412698e-4f);
+  p = fmaf(p, z, 8.33333333e-3f);
+  p = fmaf(p, z, -1.66666667e-1f);
+  const float sr = fmaf(r * z, p, r);
+  float q = fmaf(z, -2.75573192e-7f, 2.48015873e-5f);
+  q = fmaf(q, z, -1.38888889e-3f);
+  q = fmaf(q, z, 4.16666667e-2f);
+  q = fmaf(q, z, -0.5f);
+  const float cr = fmaf(q, z, 1.f);
+  const uint32_t k = static_cast<uint32_t>(static_cast<int>(n));
+  s = __uint_as_float(__float_as_uint(k & 1 ? cr : sr) ^ ((k & 2) << 30));
+  c = __uint_as_float(__float_as_uint(k & 1 ? sr : cr) ^ (((k + 1) & 2) << 30));
+}
+// ``slow``: some lane's phase may reach kSincosMax (or is NaN); the same in the wavefront
+__device__ __forceinline__ void coeff_sincos(float x, bool slow, float& s, float& c) {
+  if (slow) sincosf(x, &s, &c);
+  else sincos_reduced(x, s, c);
+}
+
+// e^-x of a finite x >= 0
+__device__ __forceinline__ float exp_neg(float x) {
+  const float t = x * -1.44269502f;  // -log2 e, and its remainder below
+  const float lo = fmaf(x, -1.92596303e-8f, fmaf(x, -1.44269502f, -t));
+  const float n = rintf(t);
+  return ldexpf(__builtin_amdgcn_exp2f((t - n) + lo), static_cast<int>(n));
+}
+
+// e_mk for one peak (the caller normalises); den = 2 s_m², rden = 1 / den: the
+// quotient with one correction step is the division's but for rare last bits
+__device__ __forceinline__ float coeff_e(const float* logw, int k, float mu, float den, float rden) {
+  const float d = logw[k] - mu, dd = d * d;
+  const float q = dd * rden;
+  return exp_neg(fmaf(fmaf(-q, den, dd), rden, q));
+}
+
+// the largest |ω_k| (uniform)
+template <int KK>
+__device__ __forceinline__ float max_omega(const float* omegas, int K) {
+  float m = 0.f;
+#pragma unroll
+  for (int k = 0; k < KK; ++k)
+    if (k < K) m = fmaxf(m, fabsf(omegas[k]));
+  return m;
 }
 
 }  // namespace
@@ -122,6 +175,7 @@ __global__ __launch_bounds__(kCoeffThreads) void coeff_fwd_kernel(
     float* __restrict__ w_out, double* __restrict__ partial) {
   const int m = threadIdx.x % kCoeffGroup;
   double r_omega = 0.0, r_ent = 0.0, r_edge = 0.0, r_b = 0.0;  // this lane's regulariser terms
+  const float om_max = max_omega<KK>(omegas, p.K);
   for (int pass = 0; pass < kCoeffPasses; ++pass) {
     const int64_t row_id = (static_cast<int64_t>(blockIdx.x) * kCoeffPasses + pass) * kCoeffRows +
                            threadIdx.x / kCoeffGroup;
@@ -136,10 +190,12 @@ __global__ __launch_bounds__(kCoeffThreads) void coeff_fwd_kernel(
     float om = 0.f;  // Σ_k ω_k² a_mk² of this peak
     {
       float e[KK], S = 0.f;
+      const float den = 2.f * (R.sg * R.sg), rden = 1.f / den;
+      const bool slow = __any(!(om_max * fabsf(R.ds) < kSincosMax));
   #pragma unroll
       for (int k = 0; k < KK; ++k) {
         if (k >= K) break;
-        e[k] = coeff_e(logw, k, R.mu, R.sg);
+        e[k] = coeff_e(logw, k, R.mu, den, rden);
         S += e[k];
       }
       const float inv = 1.f / (S + p.eps);
@@ -148,7 +204,7 @@ __global__ __launch_bounds__(kCoeffThreads) void coeff_fwd_kernel(
         if (k >= K) break;
         const float a = e[k] * inv;
         float sn, cn;
-        sincosf(omegas[k] * R.ds, &sn, &cn);
+        coeff_sincos(omegas[k] * R.ds, slow, sn, cn);
         const float w = act ? R.pi * a : 0.f;
         cc[k] = grp_sum(w * cn);
         cs[k] = grp_sum(w * sn);
@@ -334,10 +390,12 @@ __global__ __launch_bounds__(kCoeffThreads) void coeff_bwd_kernel(
   if (g_dm && m == R.amax) gds += g_dm[row];
   {
     float e[KK], a[KK], ga[KK], S = 0.f;
+    const float den = 2.f * (R.sg * R.sg), rden = 1.f / den;
+    const bool slow = __any(!(max_omega<KK>(omegas, K) * fabsf(R.ds) < kSincosMax));
 #pragma unroll
     for (int k = 0; k < KK; ++k) {
       if (k >= K) break;
-      e[k] = coeff_e(logw, k, R.mu, R.sg);
+      e[k] = coeff_e(logw, k, R.mu, den, rden);
       S += e[k];
     }
     const float inv = 1.f / (S + p.eps);
@@ -347,7 +405,7 @@ __global__ __launch_bounds__(kCoeffThreads) void coeff_bwd_kernel(
       if (k >= K) break;
       a[k] = e[k] * inv;
       float sn, cn;
-      sincosf(omegas[k] * R.ds, &sn, &cn);
+      coeff_sincos(omegas[k] * R.ds, slow, sn, cn);
       const float G = gcc[k] * cn + gcs[k] * sn;
       gpim += a[k] * G;
       ga[k] = R.pi * G + c_om * omegas[k] * omegas[k] * a[k];
@@ -360,14 +418,14 @@ __global__ __launch_bounds__(kCoeffThreads) void coeff_bwd_kernel(
 #pragma unroll
     for (int k = 0; k < KK; ++k)
       if (k < K) dot += ga[k] * a[k];
-    const float is2 = 1.f / (R.sg * R.sg);
+    const float is2 = 1.f / (R.sg * R.sg), is3 = is2 / R.sg;
 #pragma unroll
     for (int k = 0; k < KK; ++k) {
       if (k >= K) break;
       const float ge = (ga[k] - dot) * inv * e[k];
       const float d = logw[k] - R.mu;
       gmu += ge * d * is2;
-      gsg += ge * d * d * is2 / R.sg;
+      gsg += ge * d * d * is3;
     }
   }
   if (g_w) {
