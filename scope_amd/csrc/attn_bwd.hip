@@ -751,6 +751,50 @@ __device__ __forceinline__ void dkv_tile(const AttnArgs& a, const DkvBuf<MODE>& 
   }
 }
 
+// kv-major kernels: takes the q-blocks without a row that sees one of the 128
+// keys from kv0 (see drop_masked_blocks) out of the workgroup's entries
+// qbs, dse, epos (and ebias), whose order stays, and returns how many are left.
+// Every wavefront tests all entries (ne <= 64), so all come to the same
+// answers.  A dropped entry's pair-bias gradient is 0.  The caller's barrier
+// before it makes the entries readable; so they are after it.
+template <int BS, int NW, bool DP>
+__device__ __forceinline__ int drop_masked_rows(const AttnArgs& a, int ne, int h, int zpart, int64_t kv0, int* qbs,
+                                                int* dse, int* epos, float* ebias, int tid) {
+  static_assert(kChunkMax <= 64, "one wavefront holds a work item's entries");
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const bool far = lane < ne && dse[lane] > kv0 + 127;
+  if (__ballot(far) == 0) return ne;
+  int lo, hi;
+  doc_range<128>(a.docs + kv0, lane, lo, hi);
+  __syncthreads();  // every wavefront has tested the entries
+  for (int e = wave; e < ne; e += NW) {
+    const int qb = __builtin_amdgcn_readfirstlane(qbs[e]);
+    if (dse[e] > kv0 + 127 && no_doc_in<BS>(a.docs + static_cast<int64_t>(qb) * BS, lane, lo, hi) && lane == 0)
+      qbs[e] = -1 - qb;
+  }
+  __syncthreads();
+  int qb = -1, ds = 0, ep = -1;
+  float eb = 0.f;
+  if (lane < ne) {
+    qb = qbs[lane], ds = dse[lane], ep = epos[lane];
+    if (ebias) eb = ebias[lane];
+  }
+  const uint64_t kept = __ballot(qb >= 0);
+  __syncthreads();  // every entry is in registers
+  if (wave == 0 && lane < ne) {
+    if (qb >= 0) {
+      const int to = __popcll(kept & ((1ull << lane) - 1));
+      qbs[to] = qb, dse[to] = ds, epos[to] = ep;
+      if (ebias) ebias[to] = eb;
+    } else if (DP && ep >= 0) {
+      const int64_t row = static_cast<int64_t>(h) * a.QB + (-1 - qb);
+      a.dpair[(static_cast<int64_t>(zpart) * a.H * a.QB + row) * a.maxkv + ep] = 0.f;
+    }
+  }
+  __syncthreads();
+  return __popcll(kept);
+}
+
 template <int BS, int MODE, bool DP>
 __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(AttnArgs a, KvPlan pl) {
   constexpr int D = 128;
@@ -793,7 +837,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(AttnArgs a, KvPlan pl
   const int CH = pl.chunk;
   const int nch = max(1, (nq + CH - 1) / CH);
   const int i0 = chunk * CH, i1 = min(nq, i0 + CH);
-  const int ne = max(0, i1 - i0);
+  int ne = max(0, i1 - i0);
   const int32_t* ql = a.q_list + static_cast<int64_t>(h) * a.QB * a.maxkv + qo[kb];
 
   const int tid = threadIdx.x;
@@ -803,12 +847,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(AttnArgs a, KvPlan pl
   const int64_t wkv = wkv_lo + lr;
   const int krow = zpart * 128 + wave * 32 + lr;  // key row within the block
   const int64_t hT = static_cast<int64_t>(h) * a.T;
-
-  // The q-list is ascending, so only its first entry can be the diagonal
-  // block; there the query sub-tiles that end before kv0 are skipped.
-  const int qb_first = ne > 0 ? ql[i0] : 0;
-  const int skip0 = ne > 0 && qb_first == kb ? (zpart * 128) / BM : 0;
-  const int n_it = ne * NS - skip0;
 
   if (tid < ne) {
     const int qb = ql[i0 + tid];
@@ -824,9 +862,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(AttnArgs a, KvPlan pl
     epos[tid] = pos;
   }
   for (int t = tid; DP && t < CH * 4; t += blockDim.x) pslot[t / 4][t % 4] = 0.f;
+  __syncthreads();  // the entries
+  ne = drop_masked_rows<BS, 4, DP>(a, ne, h, zpart, kv0, qbs, dse, epos, ebias, tid);
+  // The q-list is ascending, so only its first entry can be the diagonal
+  // block; there the query sub-tiles that end before kv0 are skipped.
+  const int qb_first = ne > 0 ? __builtin_amdgcn_readfirstlane(qbs[0]) : 0;
+  const int skip0 = ne > 0 && qb_first == kb ? (zpart * 128) / BM : 0;
+  const int n_it = ne * NS - skip0;
   // block-mode table row of distance qb - kb (clamped: a later key block is fully masked anyway)
   for (int t = tid; MODE == 1 && t < ne * 16; t += blockDim.x) {
-    const int r = min(max(ql[i0 + t / 16] - kb, 0), NB - 1);
+    const int r = min(max(qbs[t / 16] - kb, 0), NB - 1);
     tabs[t] = static_cast<const float*>(a.table)[static_cast<int64_t>(r) * 16 + t % 16];
   }
   if (n_it > 0) {
@@ -1168,7 +1213,7 @@ __global__ __launch_bounds__(512) void attn_bwd_dkv16_kernel(AttnArgs a, KvPlan 
   const int CH = pl.chunk;
   const int nch = max(1, (nq + CH - 1) / CH);
   const int i0 = chunk * CH, i1 = min(nq, i0 + CH);
-  const int ne = max(0, i1 - i0);
+  int ne = max(0, i1 - i0);
   const int32_t* ql = a.q_list + static_cast<int64_t>(h) * a.QB * a.maxkv + qo[kb];
 
   const int tid = threadIdx.x;
@@ -1179,10 +1224,6 @@ __global__ __launch_bounds__(512) void attn_bwd_dkv16_kernel(AttnArgs a, KvPlan 
   const int krow = zpart * 128 + wave * 16 + c;  // key row within the block
   const int64_t hT = static_cast<int64_t>(h) * a.T;
 
-  const int qb_first = ne > 0 ? ql[i0] : 0;
-  const int skip0 = ne > 0 && qb_first == kb ? (zpart * 128) / BM : 0;
-  const int n_it = ne * NS - skip0;
-
   if (tid < ne) {
     const int qb = ql[i0 + tid];
     qbs[tid] = qb;
@@ -1191,7 +1232,11 @@ __global__ __launch_bounds__(512) void attn_bwd_dkv16_kernel(AttnArgs a, KvPlan 
     epos[tid] = pl.q_pos[static_cast<int64_t>(h) * a.QB * a.maxkv + qo[kb] + i0 + tid];
   }
   for (int t = tid; DP && t < CH * 8; t += blockDim.x) pslot[t / 8][t % 8] = 0.f;
-  __syncthreads();  // qbs, epos
+  __syncthreads();  // the entries
+  ne = drop_masked_rows<BS, 8, DP>(a, ne, h, zpart, kv0, qbs, dse, epos, nullptr, tid);
+  const int qb_first = ne > 0 ? __builtin_amdgcn_readfirstlane(qbs[0]) : 0;
+  const int skip0 = ne > 0 && qb_first == kb ? (zpart * 128) / BM : 0;
+  const int n_it = ne * NS - skip0;
   // the offsets of tile j (q-block qbs[e], rows (f % NS)·64 .. +63 of the list entry)
   auto tile_rof = [&](int j) __attribute__((always_inline)) -> const float* {
     if constexpr (MODE >= 2) return nullptr;  // token modes: per-row constants, no stored offsets
@@ -1416,9 +1461,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int n = min(a.kv_num[lrow], a.maxkv);  // maxkv <= kListLds
   const int32_t* lst = a.kv_idx + lrow * a.maxkv;
   for (int t = tid; t < min(n, kListLds); t += NT) kbs[t] = lst[t];
+  const int ds_end = a.ds_tok_end[qb];
   const bool pbias = a.pair_bias != nullptr;
   if (pbias)
     for (int t = tid; t < min(n, kListLds); t += NT) kbias[t] = a.pair_bias[lrow * a.maxkv + t] * kLog2e;
+  drop_masked_blocks<BS, 128, NT>(a, kbs, lst, min(n, kListLds), q0, ds_end, tid);
 
   // Q and dO of this lane's row, k-step ks: columns 32g + 8ks .. +7 (the order of the row reads)
   uint4 qreg[4], doreg[4];
@@ -1478,7 +1525,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       wd = a.width[hT + row];
     }
   }
-  const int ds_end = a.ds_tok_end[qb];
   const TileOffs16 to = tile_offs16(lane);
 
   f32x4_t dqT[8];  // dQ^T: D rows 16·md + 4g + r, this lane's query row

@@ -164,11 +164,15 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
   }
   const int32_t* lst = a.kv_idx + lrow * a.maxkv;
   for (int t = e0 + tid; t < min(n, kListLds); t += NT) kbs[t] = lst[t];
+  const int ds_end = a.ds_tok_end[qb];
   const bool pbias = a.pair_bias != nullptr;
   if (pbias)
     for (int t = e0 + tid; t < min(n, kListLds); t += NT) kbias[t] = a.pair_bias[lrow * a.maxkv + t] * kLog2e;
   if (MASS)
     for (int t = tid; t < n * NW; t += NT) mslot[t] = 0.f;  // n <= kListLds (checked on the host)
+
+  // (the other kinds report every entry)
+  if (PV) drop_masked_blocks<BS, BS, NT>(a, kbs, lst, min(n, kListLds), q0, ds_end, tid);
 
   const TileOffs to = tile_offs(lane);
   uint4 qreg[8];
@@ -197,7 +201,6 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
       R.wd = a.width[hT + R.row];
     }
   }
-  const int ds_end = a.ds_tok_end[qb];
   R.doc = a.docs[R.row];
 
   f32x16_t o[4];
