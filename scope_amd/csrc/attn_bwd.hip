@@ -20,11 +20,9 @@
 // Pass B (kv-major, one workgroup per (head, 128 keys of a key block, chunk)):
 //   dK, dV over the q-list; a block with one chunk writes bf16 directly,
 //   longer lists write fp32 partials that a reduce kernel sums in chunk order
-//   (deterministic, no floating-point atomics).  Every mode but the gated
-//   token mode runs 16 keys per wavefront on v_mfma_f32_16x16x32_bf16, eight
-//   wavefronts in two staggered groups (attn_bwd_dkv16_kernel); the gated
-//   token mode runs 32 keys per wavefront on the 32x32x16 form, four
-//   wavefronts (attn_bwd_dkv_kernel).
+//   (deterministic, no floating-point atomics).  Every mode runs 16
+//   keys per wavefront on v_mfma_f32_16x16x32_bf16, eight wavefronts in two
+//   staggered groups (attn_bwd_dkv16_kernel).
 #include <math.h>
 
 #include <algorithm>
@@ -573,193 +571,15 @@ __device__ __forceinline__ void dkv_issue(const AttnArgs& a, int h, int64_t hT, 
   for (int part = 0; part < 10; ++part) dkv_issue_part<MODE>(a, h, hT, q0, rof, b, tid, part);
 }
 
-// P and dS of register quad (mq, rq) of one tile as bf16 B operands (k index:
-// the 64 query rows): the quad is k-step 2·mq + rq/2, slots 4·(rq%2) .. +3.
-// MASK applies the causal and document masks.
-template <int MODE, bool MASK, bool DP>
-__device__ __forceinline__ void dkv_probs_quad(const AttnArgs& a, const DkvBuf<MODE>& b, const float* offw, int q0,
-                                               int lane, int wkv, int doc_kv, const f32x16_t (&s)[2],
-                                               const f32x16_t (&dp)[2], uint4 (&pb)[4], uint4 (&dsb)[4], int mq,
-                                               int rq, float& dsum) {
-  constexpr bool TOK = MODE >= 2, GATE = MODE == 3;
-  const int g = lane >> 5;
-  const int* docq = reinterpret_cast<const int*>(b.ra + 128);
-  const float cs = a.scale_log2;
-  const float glam = a.beta_log2 * a.ramp_lambda;
-  const float slsc = TOK ? 1.f : 0.f;  // b.rc holds β·slope (zero without the slope term)
-  const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? kLn2 : 0.f;
-  const int qi0 = mq * 32 + 8 * rq + 4 * g;  // 4 consecutive query rows of this register quad
-  const float4 of4 = *reinterpret_cast<const float4*>(&offw[qi0]);
-  const float4 dl4 = *reinterpret_cast<const float4*>(&b.ra[64 + qi0]);
-  const float ofv[4] = {of4.x, of4.y, of4.z, of4.w};
-  const float dlv[4] = {dl4.x, dl4.y, dl4.z, dl4.w};
-  int dcv[4] = {0, 0, 0, 0};
-  if (MASK) {
-    const int4 dc4 = *reinterpret_cast<const int4*>(&docq[qi0]);
-    dcv[0] = dc4.x;
-    dcv[1] = dc4.y;
-    dcv[2] = dc4.z;
-    dcv[3] = dc4.w;
-  }
-  float pv[4], dsv[4];
-#pragma unroll
-  for (int i2 = 0; i2 < 4; ++i2) {
-    const int r = 4 * rq + i2;
-    const int q = q0 + qi0 + i2;
-    float xv;
-    if (TOK) {
-      // slope and gate terms; softplus(x) = max(x,0) + ln2·log2(1 + 2^(-|x|·log2 e))
-      const float df = static_cast<float>(q - wkv);
-      float e = slsc * b.rc[qi0 + i2] * df;
-      if (GATE) {
-        const float xx = (fabsf(df - b.rc[64 + qi0 + i2]) - b.rc[128 + qi0 + i2]) * a.inv_tau;
-        const float sp = __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(xx) * kLog2e));
-        e -= glam * fmaf(spw, sp, fmaxf(xx, 0.f));
-      }
-      xv = fmaf(s[mq][r], cs, e + ofv[i2]);
-    } else {
-      xv = fmaf(s[mq][r], cs, ofv[i2]);
-    }
-    if (MASK) xv = mask_score(xv, wkv, q, doc_kv, dcv[i2]);
-    const float p = __builtin_amdgcn_exp2f(xv);
-    pv[i2] = p;
-    dsv[i2] = p * (dp[mq][r] + dlv[i2]);  // dlv holds -Δ
-    if (DP) dsum += dsv[i2];
-  }
-  const int ksx = 2 * mq + rq / 2;
-  const uint32_t p01 = cvt_pk_bf16(pv[0], pv[1]), p23 = cvt_pk_bf16(pv[2], pv[3]);
-  const uint32_t d01 = cvt_pk_bf16(dsv[0], dsv[1]), d23 = cvt_pk_bf16(dsv[2], dsv[3]);
-  if (rq % 2 == 0) {
-    pb[ksx].x = p01;
-    pb[ksx].y = p23;
-    dsb[ksx].x = d01;
-    dsb[ksx].y = d23;
-  } else {
-    pb[ksx].z = p01;
-    pb[ksx].w = p23;
-    dsb[ksx].z = d01;
-    dsb[ksx].w = d23;
-  }
-}
-
-// Per-row exponent offsets of a tile (lane = row), private to the wavefront.
-template <int MODE>
-__device__ __forceinline__ void dkv_offsets(const AttnArgs& a, const DkvBuf<MODE>& b, float* offw, const float* tab,
-                                            float eb, int lane) {
-  static_assert(MODE >= 2, "modes 0/1 read the offsets the q-major pass stored");
-  offw[lane] = b.ra[lane] + eb;  // the row's offset (-β·b0 - lse, or -inf) and the pair bias
-}
-
-// One 64-row query tile against this wavefront's 32 keys: S, dP, then
-// dV^T += dO^T·P and dK^T += Q^T·dS.  The copies of the next tile are issued
-// by the caller, before this tile's reads.
-template <int BS, int MODE, bool DP>
-__device__ __forceinline__ void dkv_tile(const AttnArgs& a, const DkvBuf<MODE>& b, bool masked, float* offw,
-                                         const float* tab, float eb,
-                                         int64_t q0, int lane, int64_t wkv_lo, int doc_kv,
-                                         const uint4 (&kreg)[8], const uint4 (&vreg)[8], const uint4& kf,
-                                         const uint4& kfl, f32x16_t (&dvT)[4], f32x16_t (&dkT)[4],
-                                         const TileOffs& to, float* slot) {
-  const int g = lane >> 5, lr = lane & 31;
-  const int wkv = static_cast<int>(wkv_lo) + lr;
-  dkv_offsets<MODE>(a, b, offw, tab, eb, lane);
-  // S and dP, query rows in two 32-row blocks (A operand), keys as columns (B)
-  f32x16_t s[2], dp[2];
-#pragma unroll
-  for (int mq = 0; mq < 2; ++mq) {
-    s[mq] = zero16();
-    dp[mq] = zero16();
-  }
-  // four independent accumulator chains; the A operands of k-step ks+1 are
-  // read from LDS while k-step ks runs (the fences stop the compiler from
-  // hoisting every read, which would exhaust the registers)
-  uint4 qa0 = lds_row8_o(b.q, to, 0, 0), qa1 = lds_row8_o(b.q, to, 32, 0);
-  uint4 da0 = lds_row8_o(b.d, to, 0, 0), da1 = lds_row8_o(b.d, to, 32, 0);
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    uint4 qn0 = qa0, qn1 = qa1, dn0 = da0, dn1 = da1;
-    if (ks < 7) {
-      qn0 = lds_row8_o(b.q, to, 0, ks + 1);
-      qn1 = lds_row8_o(b.q, to, 32, ks + 1);
-      dn0 = lds_row8_o(b.d, to, 0, ks + 1);
-      dn1 = lds_row8_o(b.d, to, 32, ks + 1);
-    }
-    s[0] = mfma32(qa0, kreg[ks], s[0]);
-    dp[0] = mfma32(da0, vreg[ks], dp[0]);
-    s[1] = mfma32(qa1, kreg[ks], s[1]);
-    dp[1] = mfma32(da1, vreg[ks], dp[1]);
-    // the next k-step's reads go out before this k-step's MFMAs
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    qa0 = qn0, qa1 = qn1, da0 = dn0, da1 = dn1;
-  }
-  if (MODE >= 2) {
-    const uint16_t* qf = reinterpret_cast<const uint16_t*>(b.rb);
-#pragma unroll
-    for (int mq = 0; mq < 2; ++mq) {
-      const uint4 qh = lds_row8_32(qf, mq * 32 + lr, g * 8);
-      const uint4 qlo = lds_row8_32(qf, mq * 32 + lr, 16 + g * 8);
-      s[mq] = mfma32(qh, kf, s[mq]);
-      s[mq] = mfma32(qlo, kf, s[mq]);
-      s[mq] = mfma32(qh, kfl, s[mq]);
-    }
-  }
-  uint4 pb[4], dsb[4];
-  float dsum = 0.f;
-  if (MODE >= 2 || masked) {  // token modes always take the masked form (one copy of their longer code)
-#pragma unroll
-    for (int mq = 0; mq < 2; ++mq)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq)
-        dkv_probs_quad<MODE, true, DP>(a, b, offw, static_cast<int>(q0), lane, wkv, doc_kv, s, dp, pb, dsb, mq, rq,
-                                       dsum);
-  } else {
-#pragma unroll
-    for (int mq = 0; mq < 2; ++mq)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq)
-        dkv_probs_quad<MODE, false, DP>(a, b, offw, static_cast<int>(q0), lane, wkv, doc_kv, s, dp, pb, dsb, mq, rq,
-                                        dsum);
-  }
-  if (DP) {
-    dsum = wave_sum(dsum);
-    if (lane == 0) *slot += dsum;
-  }
-  // dV^T += dO^T P,  dK^T += Q^T dS  (k index: the 64 query rows); a step is
-  // two MFMAs, so the operands are read TPD steps ahead into a ring
-  __builtin_amdgcn_sched_barrier(0);
-  constexpr int TPD = 3;
-  uint4 ta[TPD + 1], tb[TPD + 1];
-#pragma unroll
-  for (int i = 0; i < TPD; ++i) {
-    ta[i] = lds_kmajor_o(b.d, to, 16 * (i / 4), i % 4);
-    tb[i] = lds_kmajor_o(b.q, to, 16 * (i / 4), i % 4);
-  }
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int s4 = st / 4, md = st % 4;
-    if (st + TPD < 16) {
-      ta[(st + TPD) % (TPD + 1)] = lds_kmajor_o(b.d, to, 16 * ((st + TPD) / 4), (st + TPD) % 4);
-      tb[(st + TPD) % (TPD + 1)] = lds_kmajor_o(b.q, to, 16 * ((st + TPD) / 4), (st + TPD) % 4);
-    }
-    dvT[md] = mfma32(ta[st % (TPD + 1)], pb[s4], dvT[md]);
-    dkT[md] = mfma32(tb[st % (TPD + 1)], dsb[s4], dkT[md]);
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
 // kv-major kernels: takes the q-blocks without a row that sees one of the 128
 // keys from kv0 (see drop_masked_blocks) out of the workgroup's entries
-// qbs, dse, epos (and ebias), whose order stays, and returns how many are left.
+// qbs, dse, epos, whose order stays, and returns how many are left.
 // Every wavefront tests all entries (ne <= 64), so all come to the same
 // answers.  A dropped entry's pair-bias gradient is 0.  The caller's barrier
 // before it makes the entries readable; so they are after it.
 template <int BS, int NW, bool DP>
 __device__ __forceinline__ int drop_masked_rows(const AttnArgs& a, int ne, int h, int zpart, int64_t kv0, int* qbs,
-                                                int* dse, int* epos, float* ebias, int tid) {
+                                                int* dse, int* epos, int tid) {
   static_assert(kChunkMax <= 64, "one wavefront holds a work item's entries");
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const bool far = lane < ne && dse[lane] > kv0 + 127;
@@ -774,18 +594,13 @@ __device__ __forceinline__ int drop_masked_rows(const AttnArgs& a, int ne, int h
   }
   __syncthreads();
   int qb = -1, ds = 0, ep = -1;
-  float eb = 0.f;
-  if (lane < ne) {
-    qb = qbs[lane], ds = dse[lane], ep = epos[lane];
-    if (ebias) eb = ebias[lane];
-  }
+  if (lane < ne) qb = qbs[lane], ds = dse[lane], ep = epos[lane];
   const uint64_t kept = __ballot(qb >= 0);
   __syncthreads();  // every entry is in registers
   if (wave == 0 && lane < ne) {
     if (qb >= 0) {
       const int to = __popcll(kept & ((1ull << lane) - 1));
       qbs[to] = qb, dse[to] = ds, epos[to] = ep;
-      if (ebias) ebias[to] = eb;
     } else if (DP && ep >= 0) {
       const int64_t row = static_cast<int64_t>(h) * a.QB + (-1 - qb);
       a.dpair[(static_cast<int64_t>(zpart) * a.H * a.QB + row) * a.maxkv + ep] = 0.f;
@@ -795,193 +610,16 @@ __device__ __forceinline__ int drop_masked_rows(const AttnArgs& a, int ne, int h
   return __popcll(kept);
 }
 
-template <int BS, int MODE, bool DP>
-__global__ __launch_bounds__(256) void attn_bwd_dkv_kernel(AttnArgs a, KvPlan pl) {
-  constexpr int D = 128;
-  constexpr int BM = 64;  // query rows per staged tile
-  constexpr int NS = BS / BM;
-
-  __shared__ DkvBuf<MODE> buf0, buf1;
-  __shared__ __attribute__((aligned(16))) float offw[4][BM];
-  __shared__ __attribute__((aligned(16))) float tabs[MODE == 1 ? kChunkMax * 16 : 4];
-  __shared__ int qbs[kChunkMax], dse[kChunkMax], epos[kChunkMax];
-  __shared__ float ebias[kChunkMax];
-  __shared__ float pslot[kChunkMax][4];  // pair-bias gradient: per entry and wavefront
-
-  constexpr int P = BS / 128;  // workgroups (128 keys each) per key block
-  const int NB = a.QB;
-  // 1-D grid, XCD-aware: the hardware deals workgroup ids round-robin over the
-  // 8 XCDs, so id L runs on XCD L % 8.  Each XCD takes a contiguous range of
-  // (head, item) pairs, and the P parts of one item get consecutive slots on
-  // the same XCD: they read the same query tiles, which then come from its L2.
-  const int L = blockIdx.x;
-  const int per_xcd = gridDim.x / 8 / P;  // items per XCD (the grid is a multiple of 8·P)
-  const int pair = (L / 8) / P, zpart = (L / 8) % P;
-  const int item = (L % 8) * per_xcd + pair;
-  if (item >= a.H * pl.max_items) return;
-  const int h = item / pl.max_items;
-  const int x = item % pl.max_items;
-  const int32_t* its = pl.items_start + static_cast<int64_t>(h) * (NB + 1);
-  if (x >= its[NB]) return;
-  // key block owning item x: largest kb with its[kb] <= x
-  int lo = 0, hi = NB - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) / 2;
-    if (its[mid] <= x) lo = mid;
-    else hi = mid - 1;
-  }
-  const int kb = lo;
-  const int chunk = x - its[kb];
-  const int32_t* qo = a.q_off + static_cast<int64_t>(h) * (NB + 1);
-  const int nq = qo[kb + 1] - qo[kb];
-  const int CH = pl.chunk;
-  const int nch = max(1, (nq + CH - 1) / CH);
-  const int i0 = chunk * CH, i1 = min(nq, i0 + CH);
-  int ne = max(0, i1 - i0);
-  const int32_t* ql = a.q_list + static_cast<int64_t>(h) * a.QB * a.maxkv + qo[kb];
-
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid % 64, g = lane / 32, lr = lane % 32;
-  const int64_t kv0 = static_cast<int64_t>(kb) * BS + zpart * 128;  // first key row of this workgroup
-  const int64_t wkv_lo = kv0 + wave * 32;
-  const int64_t wkv = wkv_lo + lr;
-  const int krow = zpart * 128 + wave * 32 + lr;  // key row within the block
-  const int64_t hT = static_cast<int64_t>(h) * a.T;
-
-  if (tid < ne) {
-    const int qb = ql[i0 + tid];
-    qbs[tid] = qb;
-    dse[tid] = a.ds_tok_end[qb];
-    float eb = 0.f;
-    int pos = -1;
-    if (pl.q_pos) {
-      pos = pl.q_pos[static_cast<int64_t>(h) * a.QB * a.maxkv + qo[kb] + i0 + tid];
-      if (a.pair_bias && pos >= 0) eb = a.pair_bias[(static_cast<int64_t>(h) * a.QB + qb) * a.maxkv + pos] * kLog2e;
-    }
-    ebias[tid] = eb;
-    epos[tid] = pos;
-  }
-  for (int t = tid; DP && t < CH * 4; t += blockDim.x) pslot[t / 4][t % 4] = 0.f;
-  __syncthreads();  // the entries
-  ne = drop_masked_rows<BS, 4, DP>(a, ne, h, zpart, kv0, qbs, dse, epos, ebias, tid);
-  // The q-list is ascending, so only its first entry can be the diagonal
-  // block; there the query sub-tiles that end before kv0 are skipped.
-  const int qb_first = ne > 0 ? __builtin_amdgcn_readfirstlane(qbs[0]) : 0;
-  const int skip0 = ne > 0 && qb_first == kb ? (zpart * 128) / BM : 0;
-  const int n_it = ne * NS - skip0;
-  // block-mode table row of distance qb - kb (clamped: a later key block is fully masked anyway)
-  for (int t = tid; MODE == 1 && t < ne * 16; t += blockDim.x) {
-    const int r = min(max(qbs[t / 16] - kb, 0), NB - 1);
-    tabs[t] = static_cast<const float*>(a.table)[static_cast<int64_t>(r) * 16 + t % 16];
-  }
-  if (n_it > 0) {
-    const int64_t q0 = static_cast<int64_t>(qb_first) * BS + (skip0 % NS) * BM;
-    dkv_issue<MODE>(a, h, hT, q0, nullptr, buf0, tid);
-  }
-
-  uint4 kreg[8], vreg[8];
-  {
-    const uint16_t* kp = a.k + h * a.k_sh + wkv * a.k_st + g * 8;
-    const uint16_t* vp = a.v + h * a.v_sh + wkv * a.v_st + g * 8;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      kreg[ks] = *reinterpret_cast<const uint4*>(kp + ks * 16);
-      vreg[ks] = *reinterpret_cast<const uint4*>(vp + ks * 16);
-    }
-  }
-  uint4 kf = make_uint4(0, 0, 0, 0), kfl = make_uint4(0, 0, 0, 0);
-  if (MODE >= 2) {
-    kf = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.table) + wkv * kTokRow + g * 8);
-    kfl = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.table) + wkv * kTokRow + 16 + g * 8);
-  }
-  const int doc_kv = a.docs[wkv];
-  const TileOffs to = tile_offs(lane);
-
-  f32x16_t dvT[4], dkT[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    dvT[i] = zero16();
-    dkT[i] = zero16();
-  }
-
-  // iteration j covers flat index f = j + skip0: list entry f / NS, sub-tile f % NS
-  auto tile_q0 = [&](int j, int& e) __attribute__((always_inline)) {
-    const int f = j + skip0;
-    e = f / NS;
-    return static_cast<int64_t>(qbs[e]) * BS + (f % NS) * BM;
-  };
-  for (int j = 0; j < n_it; j += 2) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int jj = j + half;
-      if (jj < n_it) {
-        wait_vm0();
-        __syncthreads();  // tile jj is in LDS; every wavefront is done with tile jj-1
-        int e, en;
-        if (jj + 1 < n_it) {
-          const int64_t qn = tile_q0(jj + 1, en);
-          if (half == 0) dkv_issue<MODE>(a, h, hT, qn, nullptr, buf1, tid);
-          else dkv_issue<MODE>(a, h, hT, qn, nullptr, buf0, tid);
-        }
-        const int64_t q0 = tile_q0(jj, e);
-        const float* tab = tabs + (MODE == 1 ? e * 16 : 0);
-        if (q0 + BM - 1 >= wkv_lo) {  // else every query row precedes this wavefront's keys
-          const bool masked = !((wkv_lo + 31 <= q0) && (dse[e] <= wkv_lo));
-          const DkvBuf<MODE>& bc = half == 0 ? buf0 : buf1;
-          dkv_tile<BS, MODE, DP>(a, bc, masked, offw[wave], tab, ebias[e], q0, lane, wkv_lo, doc_kv, kreg, vreg, kf,
-                                 kfl, dvT, dkT, to, &pslot[e][wave]);
-        }
-      }
-    }
-  }
-
-  if (DP) {
-    __syncthreads();  // every wavefront's slots are final
-    if (tid < ne && epos[tid] >= 0) {
-      const float t = (pslot[tid][0] + pslot[tid][1]) + (pslot[tid][2] + pslot[tid][3]);
-      const int64_t row = static_cast<int64_t>(h) * a.QB + qbs[tid];
-      a.dpair[(static_cast<int64_t>(zpart) * a.H * a.QB + row) * a.maxkv + epos[tid]] = t;
-    }
-  }
-
-  // ---- write dK = scale·dkT^T, dV = dvT^T
-  if (nch == 1) {
-    uint16_t* dkp = a.dk + h * a.k_sh + wkv * a.k_st + 4 * g;
-    uint16_t* dvp = a.dv + h * a.v_sh + wkv * a.v_st + 4 * g;
-#pragma unroll
-    for (int md = 0; md < 4; ++md)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        uint2 vk, vv;
-        vk.x = cvt_pk_bf16(dkT[md][4 * rq] * a.scale, dkT[md][4 * rq + 1] * a.scale);
-        vk.y = cvt_pk_bf16(dkT[md][4 * rq + 2] * a.scale, dkT[md][4 * rq + 3] * a.scale);
-        vv.x = cvt_pk_bf16(dvT[md][4 * rq], dvT[md][4 * rq + 1]);
-        vv.y = cvt_pk_bf16(dvT[md][4 * rq + 2], dvT[md][4 * rq + 3]);
-        *reinterpret_cast<uint2*>(dkp + md * 32 + 8 * rq) = vk;
-        *reinterpret_cast<uint2*>(dvp + md * 32 + 8 * rq) = vv;
-      }
-  } else {
-    const int64_t slot = h * pl.max_slots + pl.slots_start[static_cast<int64_t>(h) * (NB + 1) + kb] + chunk;
-    float* pk = pl.part_dk + (slot * BS + krow) * D + 4 * g;
-    float* pv = pl.part_dv + (slot * BS + krow) * D + 4 * g;
-#pragma unroll
-    for (int md = 0; md < 4; ++md)
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        *reinterpret_cast<float4*>(pk + md * 32 + 8 * rq) =
-            make_float4(dkT[md][4 * rq], dkT[md][4 * rq + 1], dkT[md][4 * rq + 2], dkT[md][4 * rq + 3]);
-        *reinterpret_cast<float4*>(pv + md * 32 + 8 * rq) =
-            make_float4(dvT[md][4 * rq], dvT[md][4 * rq + 1], dvT[md][4 * rq + 2], dvT[md][4 * rq + 3]);
-      }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// pass B, 16 keys per wavefront (modes 0 and 1)
+// pass B, 16 keys per wavefront
 // ---------------------------------------------------------------------------
 // Eight wavefronts of 16 keys share a workgroup of 128 keys, two wavefronts
 // per SIMD, so that one wavefront's probabilities run under the other's
-// matrix products.  Per 64-row query tile a wavefront computes, with
+// matrix products.  The gated mode is bound by its probabilities (about 35
+// instructions a score, four of them transcendental); its gate terms are
+// scheduled one row block at a time, or the registers of two wavefronts per
+// SIMD would not hold them.  At T=16384, H=8, lists of 14, one document it
+// takes 386 us; 32 keys per wavefront, one wavefront per SIMD, took 506.  Per 64-row query tile a wavefront computes, with
 // v_mfma_f32_16x16x32_bf16:
 //   S = Q·K^T, dP = dO·V^T   (M = 16 query rows × 4, N = its 16 keys, K and V
 //                             of those keys held in registers as B operands)
@@ -1008,13 +646,19 @@ __device__ __forceinline__ void dkv16_probs(const AttnArgs& a, const DkvBuf<MODE
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb) {
     const int qi0 = 16 * mb + 4 * g;  // rows qi0 .. qi0+3 of the tile
-    float ofv[4], slv[4] = {0.f, 0.f, 0.f, 0.f};
+    float ofv[4], slv[4] = {0.f, 0.f, 0.f, 0.f}, dmv[4], wdv[4];
     if constexpr (TOK) {
       // the rows' offsets (-β·b0 - lse) and β·slope, stored by the q-major pass
       const float4 o4 = *reinterpret_cast<const float4*>(&b.ra[qi0]);
       const float4 s4 = *reinterpret_cast<const float4*>(&b.rc[qi0]);
       ofv[0] = o4.x + eb, ofv[1] = o4.y + eb, ofv[2] = o4.z + eb, ofv[3] = o4.w + eb;
       slv[0] = s4.x, slv[1] = s4.y, slv[2] = s4.z, slv[3] = s4.w;
+      if constexpr (GATE) {
+        const float4 m4 = *reinterpret_cast<const float4*>(&b.rc[64 + qi0]);
+        const float4 w4 = *reinterpret_cast<const float4*>(&b.rc[128 + qi0]);
+        dmv[0] = m4.x, dmv[1] = m4.y, dmv[2] = m4.z, dmv[3] = m4.w;
+        wdv[0] = w4.x, wdv[1] = w4.y, wdv[2] = w4.z, wdv[3] = w4.w;
+      }
     } else {
       const float4 of4 = *reinterpret_cast<const float4*>(&offw[qi0]);
       ofv[0] = of4.x, ofv[1] = of4.y, ofv[2] = of4.z, ofv[3] = of4.w;
@@ -1031,15 +675,13 @@ __device__ __forceinline__ void dkv16_probs(const AttnArgs& a, const DkvBuf<MODE
       float x;
       if constexpr (TOK) {
         const float df = dfb + static_cast<float>(i);  // q - wkv, exact in fp32
-        float e = slv[i] * df;
+        float e = fmaf(slv[i], df, ofv[i]);
         if constexpr (GATE) {
-          // softplus(x) = max(x,0) + ln2·log2(1 + 2^(-|x|·log2 e)); relu drops the second term
-          const float xx = (fabsf(df - b.rc[64 + qi0 + i]) - b.rc[128 + qi0 + i]) * a.inv_tau;
-          const float sp = __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(xx) * kLog2e));
-          const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? kLn2 : 0.f;
-          e -= a.beta_log2 * a.ramp_lambda * fmaf(spw, sp, fmaxf(xx, 0.f));
+          const float y = gate_y(df - dmv[i], wdv[i], a.inv_tau * kLog2e);
+          const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? 1.f : 0.f;
+          e = fmaf(-a.beta_log2 * a.ramp_lambda * kLn2, gate_g(y, 1.f + gate_en(y, spw)), e);
         }
-        x = fmaf(s[mb][i], cs, e + ofv[i]);
+        x = fmaf(s[mb][i], cs, e);
       } else {
         x = fmaf(s[mb][i], cs, ofv[i]);
       }
@@ -1053,6 +695,7 @@ __device__ __forceinline__ void dkv16_probs(const AttnArgs& a, const DkvBuf<MODE
     pw[2 * mb + 1] = cvt_pk_bf16(pv[2], pv[3]);
     dw[2 * mb] = cvt_pk_bf16(dv[0], dv[1]);
     dw[2 * mb + 1] = cvt_pk_bf16(dv[2], dv[3]);
+    if constexpr (GATE) __builtin_amdgcn_sched_barrier(0);  // one row block's gate terms live at a time
   }
   pb[0] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
   pb[1] = make_uint4(pw[4], pw[5], pw[6], pw[7]);
@@ -1190,7 +833,10 @@ __global__ __launch_bounds__(512) void attn_bwd_dkv16_kernel(AttnArgs a, KvPlan 
 
   constexpr int P = BS / 128;  // workgroups (128 keys each) per key block
   const int NB = a.QB;
-  // 1-D grid, XCD-aware, as attn_bwd_dkv_kernel
+  // 1-D grid, XCD-aware: the hardware deals workgroup ids round-robin over the
+  // 8 XCDs, so id L runs on XCD L % 8.  Each XCD takes a contiguous range of
+  // (head, item) pairs, and the P parts of one item get consecutive slots on
+  // the same XCD: they read the same query tiles, which then come from its L2.
   const int L = blockIdx.x;
   const int per_xcd = gridDim.x / 8 / P;
   const int pair = (L / 8) / P, zpart = (L / 8) % P;
@@ -1233,7 +879,7 @@ __global__ __launch_bounds__(512) void attn_bwd_dkv16_kernel(AttnArgs a, KvPlan 
   }
   for (int t = tid; DP && t < CH * 8; t += blockDim.x) pslot[t / 8][t % 8] = 0.f;
   __syncthreads();  // the entries
-  ne = drop_masked_rows<BS, 8, DP>(a, ne, h, zpart, kv0, qbs, dse, epos, nullptr, tid);
+  ne = drop_masked_rows<BS, 8, DP>(a, ne, h, zpart, kv0, qbs, dse, epos, tid);
   const int qb_first = ne > 0 ? __builtin_amdgcn_readfirstlane(qbs[0]) : 0;
   const int skip0 = ne > 0 && qb_first == kb ? (zpart * 128) / BM : 0;
   const int n_it = ne * NS - skip0;
@@ -1562,8 +1208,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // probabilities and dS^T: key j = 16·kb4 + 4g + r of the tile
     const int lim = row - kv0;  // keys j <= lim are causal
     const float dfl = static_cast<float>(lim - 4 * g);
-    const bool softplus = a.gate_kind == SCOPE_GATE_SOFTPLUS;
-    const float glam = a.beta_log2 * a.ramp_lambda;
+    const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? 1.f : 0.f;
+    const float glam = a.beta_log2 * a.ramp_lambda * kLn2, y_scale = a.inv_tau * kLog2e;
     float rs = 0.f, pm = 0.f;
     uint32_t dw[8], pw[8];
     // The gated mode takes the tile's four 16-key blocks in two halves (the
@@ -1625,22 +1271,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           for (int r = 0; r < 4; ++r) {
             const int j = 16 * kb4 + 4 * g + r;
             float x;
-            float sig = 0.f, sgn = 0.f, df = 0.f;
+            float sig = 0.f, ssig = 0.f, df = 0.f;  // the gate's slope in |Δ - δ|, and in Δ - δ
             if (TOK) {
               df = dfl - static_cast<float>(16 * kb4 + r);  // lim - j, exact in fp32
-              float e = slp * df;
+              float e = fmaf(slp, df, off);
               if (GATE) {
                 const float dd = df - dm;
-                const float xx = (fabsf(dd) - wd) * a.inv_tau;
-                const float en = __builtin_amdgcn_exp2f(-fabsf(xx) * kLog2e);
-                const float inv = __builtin_amdgcn_rcpf(1.f + en);
-                const float lp = kLn2 * __builtin_amdgcn_logf(1.f + en);
-                const float gt = fmaxf(xx, 0.f) + (softplus ? lp : 0.f);
-                sig = softplus ? (xx >= 0.f ? inv : en * inv) : (xx > 0.f ? 1.f : 0.f);
-                sgn = dd > 0.f ? 1.f : (dd < 0.f ? -1.f : 0.f);
-                e -= glam * gt;
+                const float y = gate_y(dd, wd, y_scale);
+                const float en = gate_en(y, spw), en1 = 1.f + en;
+                const float inv = __builtin_amdgcn_rcpf(en1);
+                sig = y > 0.f ? inv : en * inv;
+                ssig = dd != 0.f ? copysignf(sig, dd) : 0.f;
+                e = fmaf(-glam, gate_g(y, en1), e);
               }
-              x = fmaf(s[kl][r], cs, e + off);
+              x = fmaf(s[kl][r], cs, e);
             } else {
               x = fmaf(s[kl][r], cs, off);
             }
@@ -1655,10 +1299,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
               ex[0] += d * df;
               ex[3] += p * df;
               if (GATE) {
-                ex[1] += d * sig * sgn;
-                ex[2] += d * sig;
-                ex[4] += p * sig * sgn;
-                ex[5] += p * sig;
+                ex[1] = fmaf(d, ssig, ex[1]);
+                ex[2] = fmaf(d, sig, ex[2]);
+                ex[4] = fmaf(p, ssig, ex[4]);
+                ex[5] = fmaf(p, sig, ex[5]);
               }
             }
           }
@@ -2114,11 +1758,9 @@ static void launch_bwd(const AttnArgs& a, const KvPlan& pl, int mode, int phases
   const bool dp = a.dpair != nullptr;  // the pair-bias gradient runs in its own instantiation
   if (phases & SCOPE_BWD_DKV_MAIN) {
     // 16 keys per wavefront, 8 wavefronts (two per SIMD) per 128 keys
-    // (the gated token mode spills 20-40 registers here: it keeps the
-    // 32-keys-per-wavefront kernel, one wavefront per SIMD)
     const int m = mode == SCOPE_BIAS_TOKEN ? (gate ? 3 : 2) : (mode == SCOPE_BIAS_BLOCK ? 1 : 0);
-    if (m == 3 && dp) hipLaunchKernelGGL((attn_bwd_dkv_kernel<BS, 3, true>), gk, dim3(256), 0, s, a, pl);
-    else if (m == 3) hipLaunchKernelGGL((attn_bwd_dkv_kernel<BS, 3, false>), gk, dim3(256), 0, s, a, pl);
+    if (m == 3 && dp) hipLaunchKernelGGL((attn_bwd_dkv16_kernel<BS, 3, true>), gk, dim3(512), 0, s, a, pl);
+    else if (m == 3) hipLaunchKernelGGL((attn_bwd_dkv16_kernel<BS, 3, false>), gk, dim3(512), 0, s, a, pl);
     else if (m == 2 && dp) hipLaunchKernelGGL((attn_bwd_dkv16_kernel<BS, 2, true>), gk, dim3(512), 0, s, a, pl);
     else if (m == 2) hipLaunchKernelGGL((attn_bwd_dkv16_kernel<BS, 2, false>), gk, dim3(512), 0, s, a, pl);
     else if (m == 1 && dp) hipLaunchKernelGGL((attn_bwd_dkv16_kernel<BS, 1, true>), gk, dim3(512), 0, s, a, pl);

@@ -56,12 +56,12 @@ __device__ __forceinline__ void fwd_scores(const AttnArgs& a, const Tile& b, con
   constexpr bool TOK = MODE >= 2, GATE = MODE == 3;
   const int g = lane >> 5;
   const float cs = a.scale_log2;
-  const float glam = a.beta_log2 * a.ramp_lambda;
-  const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? kLn2 : 0.f;
+  const float glam = a.beta_log2 * a.ramp_lambda * kLn2, y_scale = a.inv_tau * kLog2e;
+  const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? 1.f : 0.f;
   const int lim = R.row - kv0;  // keys j <= lim are causal
   // slope term slp·(lim - j), j = jc + 4g with jc a constant of the register:
   // fma(-slp, jc, slp·(lim - 4g)) (the integers are exact in fp32)
-  const float sbase = GATE ? 0.f : R.slp * static_cast<float>(lim - 4 * g);
+  const float dfl = static_cast<float>(lim - 4 * g), sbase = R.slp * dfl;
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -77,13 +77,11 @@ __device__ __forceinline__ void fwd_scores(const AttnArgs& a, const Tile& b, con
         const int r = 4 * rq + i, j = j0 + i;
         float x;
         if (TOK) {
-          const float df = static_cast<float>(lim - j);
-          float e = GATE ? R.slp * df : fmaf(-R.slp, static_cast<float>(mb * 32 + 8 * rq + i), sbase);
+          const float jc = static_cast<float>(mb * 32 + 8 * rq + i);
+          float e = fmaf(-R.slp, jc, sbase);
           if (GATE) {
-            // softplus(x) = max(x,0) + ln2·log2(1 + 2^(-|x|·log2 e)); relu drops the second term
-            const float xx = (fabsf(df - R.dm) - R.wd) * a.inv_tau;
-            const float sp = __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(xx) * kLog2e));
-            e -= glam * fmaf(spw, sp, fmaxf(xx, 0.f));
+            const float y = gate_y((dfl - jc) - R.dm, R.wd, y_scale);
+            e = fmaf(-glam, gate_g(y, 1.f + gate_en(y, spw)), e);
           }
           x = fmaf(s[mb][r], cs, e);
         } else {
