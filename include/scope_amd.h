@@ -168,6 +168,12 @@ int scope_pointer_bwd(const scope_ptr_bwd_params* p, const float* qbar, const fl
                       const int32_t* kv_num, const int32_t* kv_idx, const int32_t* q_off,
                       const int32_t* q_list, const float* pair_bias, const float* dpair_bias, uint16_t* dq,
                       uint16_t* dk, void* workspace, void* stream);
+/* scope_pointer_bwd with every row of dq and dk [H, T = NB·bs, D] written, not
+ * added to: their contents before the call do not matter. */
+int scope_pointer_bwd_store(const scope_ptr_bwd_params* p, const float* qbar, const float* kbar,
+                            const int32_t* kv_num, const int32_t* kv_idx, const int32_t* q_off,
+                            const int32_t* q_list, const float* pair_bias, const float* dpair_bias, uint16_t* dq,
+                            uint16_t* dk, void* workspace, void* stream);
 
 /* ------------------------------------------------------------------------
  * Transposed (q-major) lists.  Replaces BlockMask.from_kv_blocks ->

@@ -107,6 +107,7 @@ _PROTOS = {
     "scope_pointer_pair_bias": (c_int, [C.POINTER(PtrScoreParams), c_float, P, P, P, P, P, P, P, P, P]),
     "scope_pointer_bwd_workspace_bytes": (c_int64, [C.POINTER(PtrBwdParams)]),
     "scope_pointer_bwd": (c_int, [C.POINTER(PtrBwdParams)] + [P] * 12),
+    "scope_pointer_bwd_store": (c_int, [C.POINTER(PtrBwdParams)] + [P] * 12),
     "scope_transpose_workspace_bytes": (c_int64, [c_int, c_int]),
     "scope_transpose_blocks": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P]),
     "scope_transpose_blocks_noalloc": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P]),

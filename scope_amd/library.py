@@ -282,10 +282,13 @@ def soft_pointer_bwd(qbar: Tensor, kbar: Tensor, kv_num: Tensor, kv_idx: Tensor,
                      logit_scale: float, soft_temp: float) -> tuple[Tensor, Tensor]:
     """(dq, dk) bf16 with q_like's / k_like's shape and strides: the soft
     weights' gradient through the block means."""
-    dq = torch.empty_like(q_like, dtype=torch.bfloat16).zero_()
-    dk = torch.empty_like(k_like, dtype=torch.bfloat16).zero_()
+    dq = torch.empty_like(q_like, dtype=torch.bfloat16)
+    dk = torch.empty_like(k_like, dtype=torch.bfloat16)
+    store = q_like.shape[2] == k_like.shape[2] == qbar.shape[1] * bs  # the blocks cover every row
+    if not store:
+        dq.zero_(), dk.zero_()
     ops.pointer_bwd(qbar, kbar, kv_num, kv_idx, q_off, q_list, pair_bias, dpair_bias.contiguous(), dq, dk, bs=bs,
-                    logit_scale=logit_scale, soft_temp=soft_temp, check=False)
+                    logit_scale=logit_scale, soft_temp=soft_temp, check=False, store=store)
     return dq, dk
 
 

@@ -260,10 +260,11 @@ def pointer_pair_bias(kv_num: torch.Tensor, kv_idx: torch.Tensor, picks: torch.T
 def pointer_bwd(qbar: torch.Tensor, kbar: torch.Tensor, kv_num: torch.Tensor, kv_idx: torch.Tensor,
                 q_off: torch.Tensor, q_list: torch.Tensor, pair_bias: torch.Tensor, dpair_bias: torch.Tensor,
                 dq: torch.Tensor, dk: torch.Tensor, *, bs: int, logit_scale: float, soft_temp: float,
-                check: bool = True) -> None:
+                check: bool = True, store: bool = False) -> None:
     """Add the soft pointer weights' gradient path (through the block means)
-    to dq and dk [1,H,T,D] bf16 in place.  ``check``: validate kv_num /
-    kv_idx first (``check_lists``); q_off / q_list must be their transpose."""
+    to dq and dk [1,H,T,D] bf16 in place; ``store``: write it there instead.
+    ``check``: validate kv_num / kv_idx first (``check_lists``); q_off /
+    q_list must be their transpose."""
     from ._lib import PtrBwdParams
 
     dev = _gpu("pointer_bwd", qbar, kbar, kv_num, kv_idx, q_off, q_list, pair_bias, dpair_bias, dq, dk)
@@ -277,7 +278,7 @@ def pointer_bwd(qbar: torch.Tensor, kbar: torch.Tensor, kv_num: torch.Tensor, kv
                        soft_temp=float(soft_temp), q_sh=qsh, q_st=qst, k_sh=ksh, k_st=kst)
     ws = torch.empty(max(16, query("scope_pointer_bwd_workspace_bytes", C.byref(prm))), dtype=torch.uint8,
                      device=dev)
-    call("scope_pointer_bwd", C.byref(prm), _p(_f32(qbar)), _p(_f32(kbar)), _p(_i32(kv_num.reshape(H, NB))),
+    call("scope_pointer_bwd_store" if store else "scope_pointer_bwd", C.byref(prm), _p(_f32(qbar)), _p(_f32(kbar)), _p(_i32(kv_num.reshape(H, NB))),
          _p(_i32(kv_idx.reshape(H, NB, L))), _p(_i32(q_off)), _p(_i32(q_list)), _p(_f32(pair_bias)),
          _p(_f32(dpair_bias)), _p(dq), _p(dk), _p(ws), _stream(dev))
 
