@@ -290,9 +290,11 @@ __device__ __forceinline__ float bf16_round(float x) { return static_cast<float>
 // q's row r0 (a wavefront's first row; its 32 rows lie in one segment, as
 // segments are a multiple of 32 rows): the segment split once per
 // wavefront, in scalar registers
+// (in units of 32 rows: a 32-bit division is a fifth of a 64-bit one's instructions)
 __device__ __forceinline__ const uint16_t* mlp_wave_rows(const MlpArgs& g, int64_t r0) {
-  const int64_t r = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(r0 >> 5))) * 32;
-  return g.q + (r / g.seg) * g.q_ss + (r % g.seg) * g.q_rs;
+  const uint32_t r = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(r0 >> 5)));
+  const uint32_t seg = static_cast<uint32_t>(g.seg >> 5), s = r / seg;
+  return g.q + static_cast<int64_t>(s) * g.q_ss + static_cast<int64_t>(r - s * seg) * 32 * g.q_rs;
 }
 
 // A row of y or gy is O bf16 (41 for eight peaks: 82 bytes), so its chunks start
@@ -341,6 +343,30 @@ __device__ __forceinline__ void mlp_y_store(uint16_t* yp, int O, int o0, uint32_
 
 __device__ __forceinline__ float mlp_sigmoid(float z) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-z * kLog2e));
+}
+
+// two values rounded to bf16, as fp32
+__device__ __forceinline__ void bf16_round2(float& a, float& b) {
+  const uint32_t w = cvt_pk_bf16(a, b);
+  a = bf16_lo(w), b = bf16_hi(w);
+}
+
+// Two hidden units' x1 = SiLU(z1) and dz1 = SiLU'(z1)·dx1, z1 and dx1 = gy·W2
+// rounded to bf16 first (bf16 tensors in the reference).  With x1 at hand
+// SiLU'(z) = σ + x1·(1 - σ).  The VALU work of the two backward kernels is
+// here: 11 instructions and two transcendentals a unit (13 with the values
+// rounded one by one and the derivative as σ·(1 + z·(1 - σ))).  With it, the
+// 32-bit row split and db2 shared among the hidden blocks, the head at a
+// million rows, forward and backward, went from 1/1.063 to 1/1.108 of a fixed
+// older build timed beside it (1214 us on a slow box).
+__device__ __forceinline__ void mlp_silu_bwd2(float z0, float z1, float dx0, float dx1, float (&xv)[2],
+                                              float (&dv)[2]) {
+  bf16_round2(z0, z1);
+  bf16_round2(dx0, dx1);
+  const float s0 = mlp_sigmoid(z0), s1 = mlp_sigmoid(z1);
+  xv[0] = z0 * s0, xv[1] = z1 * s1;
+  dv[0] = dx0 * fmaf(xv[0], 1.f - s0, s0);
+  dv[1] = dx1 * fmaf(xv[1], 1.f - s1, s1);
 }
 
 __device__ void mlp_load_weights(const MlpArgs& g, MlpLds& L, int tid) {
@@ -431,7 +457,8 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_fwd_kernel(MlpArgs g) {
       uint32_t w[8];
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
-        const float z0 = bf16_round(z[r]), z1 = bf16_round(z[r + 1]);  // z1 is a bf16 tensor in the reference
+        float z0 = z[r], z1 = z[r + 1];
+        bf16_round2(z0, z1);  // z1 is a bf16 tensor in the reference
         w[r / 2] = cvt_pk_bf16(z0 * mlp_sigmoid(z0), z1 * mlp_sigmoid(z1));
       }
       const uint4 xp[2] = {make_uint4(w[0], w[1], w[2], w[3]), make_uint4(w[4], w[5], w[6], w[7])};
@@ -452,6 +479,8 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_fwd_kernel(MlpArgs g) {
   }
 }
 
+// INTER: x1 and dz1 are written too
+template <bool INTER>
 __global__ __launch_bounds__(kMlpThreads) void mlp_bwd_kernel(MlpArgs g) {
   __shared__ MlpLds L;
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, gq = lane / 32, lr = lane % 32;
@@ -502,18 +531,11 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_bwd_kernel(MlpArgs g) {
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         float xv[2], dv[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          // z1 and dx1 = gy·W2 are bf16 tensors in the reference
-          const float zz = bf16_round(z[r + i]);
-          const float sg = mlp_sigmoid(zz);
-          xv[i] = zz * sg;
-          dv[i] = bf16_round(dx[r + i]) * (sg * fmaf(zz, 1.f - sg, 1.f));  // SiLU'(z1)·dx1
-        }
-        xw[r / 2] = cvt_pk_bf16(xv[0], xv[1]);
+        mlp_silu_bwd2(z[r], z[r + 1], dx[r], dx[r + 1], xv, dv);
+        if (INTER) xw[r / 2] = cvt_pk_bf16(xv[0], xv[1]);
         dw[r / 2] = cvt_pk_bf16(dv[0], dv[1]);
       }
-      if (g.x1) {
+      if (INTER) {
         // x1 and dz1 rows: hidden 32hb + 8q + 4gq .. +3 in register quad q
         uint16_t* xr = g.x1 + row * kMlpH + 32 * hb + 4 * gq;
         uint16_t* dr = g.dz1 + row * kMlpH + 32 * hb + 4 * gq;
@@ -574,7 +596,7 @@ struct MlpWgradSum {
   float dw1[32 * kMlpD];      // [hidden][d]
   float dw2[32 * kMlpOMax];   // [hidden][o]
   float db1[32];
-  float db2[kMlpOMax];
+  float db2[32];              // of the hidden block's k-step and output block
 };
 static_assert(4 * sizeof(MlpWgradSum) <= sizeof(MlpWgradLds), "mlp_wgrad_kernel: the sums reuse the tile buffers");
 static_assert(kMwCopies == 4, "mlp_wgrad_kernel: the waits below count four copies per tile");
@@ -644,7 +666,7 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
   // other half of each 256-byte row stays unused), two of each per thread
   auto issue = [&](int64_t t, int buf) __attribute__((always_inline)) {
     const int64_t r0 = t * kMwTileRows;
-    const uint16_t* qb = g.q + (r0 / g.seg) * g.q_ss + (r0 % g.seg) * g.q_rs;  // a tile never spans segments
+    const uint16_t* qb = mlp_wave_rows(g, r0);  // a tile never spans segments
     const uint16_t* gb = g.gyp + r0 * kMlpOMax;
 #pragma unroll
     for (int jj = 0; jj < kMwTileRows * 16 / kMlpThreads; ++jj) {
@@ -668,8 +690,9 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc1[i] = zero16();
   acc2[0] = acc2[1] = zero16();
-  float db1 = 0.f, db2[2] = {0.f, 0.f};
-  const bool do_db2 = hb == 0;
+  // db2 on the first quad's workgroups: hidden block hl sums k-step hl / 2, output block hl % 2
+  // (on one hidden block's wavefronts alone, the others waited for them at every tile)
+  float db1 = 0.f, db2 = 0.f;
   for (int i = 0; i < kMwBufs - 1; ++i)
     if (t0 + i < t1) issue(t0 + i, i);
   for (int64_t t = t0; t < t1; ++t) {
@@ -696,13 +719,7 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
       float xv[2], dv[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float zz = bf16_round(z[r + i]);
-        const float sg = mlp_sigmoid(zz);
-        xv[i] = zz * sg;
-        dv[i] = bf16_round(dx[r + i]) * (sg * fmaf(zz, 1.f - sg, 1.f));  // SiLU'(z1)·dx1
-      }
+      mlp_silu_bwd2(z[r], z[r + 1], dx[r], dx[r + 1], xv, dv);
       xw[r / 2] = cvt_pk_bf16(xv[0], xv[1]);
       dw[r / 2] = cvt_pk_bf16(dv[0], dv[1]);
       db1 += bf16_lo(dw[r / 2]) + bf16_hi(dw[r / 2]);
@@ -717,10 +734,10 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
       for (int ob = 0; ob < 2; ++ob) {
         const uint4 gv = lds_kmajor_o(gt, to, 32 * rsub + 16 * kk, ob);
         acc2[ob] = mfma32(xa, gv, acc2[ob]);
-        if (do_db2) {
+        if (hq == 0 && hl == 2 * kk + ob) {
           const uint32_t w4[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) db2[ob] += bf16_lo(w4[j]) + bf16_hi(w4[j]);
+          for (int j = 0; j < 4; ++j) db2 += bf16_lo(w4[j]) + bf16_hi(w4[j]);
         }
       }
     }
@@ -730,8 +747,7 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
 
   // lanes l and l ^ 32 summed different rows of the same unit / column
   db1 += __shfl_xor(db1, 32, 64);
-  db2[0] += __shfl_xor(db2[0], 32, 64);
-  db2[1] += __shfl_xor(db2[1], 32, 64);
+  db2 += __shfl_xor(db2, 32, 64);
   MlpWgradSum& S = reinterpret_cast<MlpWgradSum*>(&L)[hl];
   for (int step = 0; step < 2; ++step) {
     if (rsub == step) {
@@ -751,8 +767,7 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
         }
       if (gq == 0) {
         S.db1[lr] = step == 0 ? db1 : S.db1[lr] + db1;
-        S.db2[lr] = step == 0 ? db2[0] : S.db2[lr] + db2[0];
-        S.db2[32 + lr] = step == 0 ? db2[1] : S.db2[32 + lr] + db2[1];
+        S.db2[lr] = step == 0 ? db2 : S.db2[lr] + db2;
       }
     }
     __syncthreads();
@@ -770,7 +785,7 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_wgrad_kernel(MlpArgs g, float
     p2[o * kMlpH + 128 * hq + hh] = SS[hh / 32].dw2[(hh % 32) * kMlpOMax + o];
   }
   if (tid < 128) p1[kMlpH * kMlpD + 128 * hq + tid] = SS[tid / 32].db1[tid % 32];
-  if (hq == 0 && tid < kMlpOMax) p2[kMlpOMax * kMlpH + tid] = SS[0].db2[tid];
+  if (hq == 0 && tid < kMlpOMax) p2[kMlpOMax * kMlpH + tid] = SS[tid / 32].db2[tid % 32] + SS[2 + tid / 32].db2[tid % 32];
 }
 
 }  // namespace
@@ -893,7 +908,8 @@ extern "C" int scope_coeff_mlp_bwd(const scope_mlp_params* p, const uint16_t* q,
   g.dz1 = dz1;
   g.x1 = x1;
   g.gyp = gyp;
-  hipLaunchKernelGGL(mlp_bwd_kernel, dim3(mlp_grid(p->rows)), dim3(kMlpThreads), 0, as_stream(stream), g);
+  hipLaunchKernelGGL((x1 ? mlp_bwd_kernel<true> : mlp_bwd_kernel<false>), dim3(mlp_grid(p->rows)), dim3(kMlpThreads), 0,
+                     as_stream(stream), g);
   return check_launch("MLP backward kernel");
 }
 
