@@ -305,8 +305,9 @@ __device__ __forceinline__ const uint16_t* mlp_wave_rows(const MlpArgs& g, int64
 // from 354 to 332, the weight-gradient kernel beside them unchanged (336, 359:
 // the second figure on a slower box).
 
-// Outputs 16ks + 8gq .. +7 of a row as bf16 pairs, zero past O.  Reads up to
-// 15 outputs past the end of the row; the last rows of the buffer (safe = false)
+// Outputs 16ks + 8gq .. +7 of a row as bf16 pairs; past O whatever follows
+// (up to 15 outputs), which mlp_gy_mask clears: apart, so that nothing waits
+// for the load before it is needed.  The last rows of the buffer (safe = false)
 // take single elements.
 __device__ __forceinline__ uint4 mlp_gy_chunk(const uint16_t* gp, int O, int ks, int gq, bool safe) {
   if (16 * ks >= O) return make_uint4(0, 0, 0, 0);
@@ -314,10 +315,6 @@ __device__ __forceinline__ uint4 mlp_gy_chunk(const uint16_t* gp, int O, int ks,
   uint32_t w[4];
   if (safe) {
     __builtin_memcpy(w, gp + o0, 16);
-    if (16 * ks + 16 > O) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] &= (o0 + 2 * j < O ? 0xffffu : 0u) | (o0 + 2 * j + 1 < O ? 0xffff0000u : 0u);
-    }
   } else {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -325,6 +322,17 @@ __device__ __forceinline__ uint4 mlp_gy_chunk(const uint16_t* gp, int O, int ks,
       const uint32_t lo = o < O ? gp[o] : 0u, hi = o + 1 < O ? gp[o + 1] : 0u;
       w[j] = lo | (hi << 16);
     }
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ __forceinline__ uint4 mlp_gy_mask(const uint4& v, int O, int ks, int gq) {
+  if (16 * ks + 16 <= O) return v;
+  uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int o = 16 * ks + 8 * gq + 2 * j;
+    w[j] &= (o < O ? 0xffffu : 0u) | (o + 1 < O ? 0xffff0000u : 0u);
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
@@ -488,21 +496,27 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_bwd_kernel(MlpArgs g) {
   __syncthreads();
   const TileOffs to = tile_offs(lane);
   const int64_t tiles = (g.rows + kMlpTileRows - 1) / kMlpTileRows;
+  // a tile's rows of q, and of the output gradient as B operands of dX1^T (k =
+  // outputs 16ks + 8gq .. +7, zero past O)
+  uint4 xb[8], gb[4];
+  auto load_rows = [&](int64_t t) __attribute__((always_inline)) {
+    const int64_t r0 = t * kMlpTileRows + wave * 32;
+    if (r0 >= g.rows) return;
+    const uint16_t* qp = mlp_wave_rows(g, r0) + lr * g.q_rs + 8 * gq;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) xb[ks] = *reinterpret_cast<const uint4*>(qp + 16 * ks);
+    // (the 32 rows after a wavefront's are in the buffer unless its own are the last)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) gb[ks] = mlp_gy_chunk(g.gy + (r0 + lr) * g.O, g.O, ks, gq, r0 + 32 < g.rows);
+  };
+  load_rows(blockIdx.x);
   for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
     const int64_t row = t * kMlpTileRows + wave * 32 + lr;
     if (t * kMlpTileRows + wave * 32 >= g.rows) break;
-    const uint16_t* qp = mlp_wave_rows(g, t * kMlpTileRows + wave * 32) + lr * g.q_rs + 8 * gq;
-    uint4 xb[8];
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) xb[ks] = *reinterpret_cast<const uint4*>(qp + 16 * ks);
-    // the output gradient as B operands of dX1^T (k = outputs 16ks + 8gq .. +7), zero past O;
-    // the same values padded to 64 columns for the weight gradient
-    uint4 gb[4];
-    const uint16_t* gp = g.gy + row * g.O;
+    // the output gradient padded to 64 columns, for the weight gradient
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      // (the 32 rows after a wavefront's are in the buffer unless its own are the last)
-      gb[ks] = mlp_gy_chunk(gp, g.O, ks, gq, t * kMlpTileRows + wave * 32 + 32 < g.rows);
+      gb[ks] = mlp_gy_mask(gb[ks], g.O, ks, gq);
       *reinterpret_cast<uint4*>(g.gyp + row * kMlpOMax + 16 * ks + 8 * gq) = gb[ks];
     }
     // per hidden block: Z^T and dX1^T, the VALU work, the dQ^T products (the
@@ -527,6 +541,10 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_bwd_kernel(MlpArgs g) {
     for (int hb = 0; hb < 8; ++hb) {
       f32x16_t z, dx;
       zdx(hb, z, dx);
+      // the rows' last products are issued: the next tile's take their registers, their
+      // latency under this block's VALU work and products (1M rows: 335 -> 310 us; the
+      // same in the forward, whose stores are few, changed nothing)
+      if (hb == 7) load_rows(t + gridDim.x);
       uint32_t xw[8], dw[8];
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
