@@ -61,7 +61,8 @@ def call(name: str, *args) -> None:
 
 def _stream(dev: torch.device):
     # the raw handle of torch.cuda.current_stream(dev), without building its Python object
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(dev.index))
+    # (a device without an index is the current one)
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index))
 
 
 def _gpu(name: str, *ts: torch.Tensor | None) -> torch.device:
