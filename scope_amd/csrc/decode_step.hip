@@ -37,6 +37,9 @@
 // of the process run at a time (two half-resident ones would wait for each
 // other).  Every wait ends: after spin_ticks the waiter sets the status word
 // and goes on with NaN, which reaches every row through the tagged words.
+// The lock does not reach other processes: two that step on one device at the
+// same moment may wait for each other until that limit (capacity for two such
+// kernels, 128 registers a lane, spills 93 of the 181).
 #include <math.h>
 
 #include "common.h"

@@ -151,7 +151,7 @@ class ScopeDecoder(nn.Module):
         self._g_out = None
         self._g_warm = 0
         # the one-launch step (``_fused``): the table of the layers' tensors, the
-        # addresses it was made from, and the status its waits set (pinned)
+        # addresses and layouts it was made from, and the status its waits set (pinned)
         self._step_key: tuple | None = None
         self._step_table = None
         self._step_status = None
@@ -199,6 +199,11 @@ class ScopeDecoder(nn.Module):
         bs = cfg.block_size
         if T % bs or T > self.max_len:
             raise ValueError(f"prefill: T={T} must be a multiple of {bs} and at most {self.max_len}")
+        if self._step_status is not None and int(self._step_status[0]):
+            # a wait of an earlier one-launch step expired: its workspace and the
+            # graph that uses it are left behind, once nothing runs on them
+            torch.cuda.synchronize(self.device)
+            self._graph = self._g_table = self._step_key = self._step_table = self._step_status = None
         tok = tokens.to(self.device).long()
         self.tokens[:T] = tok
         self.docs[:T] = (tok == EOT).cumsum(0).to(torch.int32)
@@ -264,10 +269,10 @@ class ScopeDecoder(nn.Module):
                 or any(lay["lambdas"] != (1.0, 0.0) for lay in self.layers) or len(self.layers) != 2 * n:
             return None
         names = ("qkv", "proj", "mlp_fc", "mlp_proj")
-        key = tuple(lay[m].data_ptr() if m in lay else 0 for lay in self.layers for m in names) \
-            + tuple(lay.get("vlam", ()) for lay in self.layers) \
-            + tuple(0 if t is None else t.data_ptr() for ts in (self.k_cache, self.v_cache, self.list_num, self.list_idx)
-                    for t in ts)
+        # (an address alone could be a later tensor of another layout)
+        key = tuple((t.data_ptr(), t.dtype, t.shape, t.stride()) if t is not None else None for ts in
+                    (*([lay.get(m) for m in names] for lay in self.layers), self.k_cache, self.v_cache, self.list_num,
+                     self.list_idx) for t in ts) + tuple(lay.get("vlam", ()) for lay in self.layers)
         if key != self._step_key:
             ve = [0, 1, 2] + [-1] * (cfg.num_layers - 6) + [0, 1, 2]
             layers = []

@@ -114,3 +114,19 @@ def test_expired_wait_gives_nan_and_raises():
     m._step_status[0] = 1
     with pytest.raises(RuntimeError, match="waited too long"):
         m.step(toks[130])
+    # the next request starts over with a workspace of its own
+    m.prefill(toks[:128])
+    m.step(toks[128])
+    assert bool(torch.isfinite(m.step(toks[129])).all())
+
+
+def test_replaced_weights_of_another_layout():
+    """A weight replaced in place of its memory by one of another layout is
+    seen: the one-launch step serves contiguous rows only."""
+    m = _model(256, True, 6, use_graph=False)
+    assert m._fused() is not None
+    w = m.layers[0]["mlp_fc"]
+    m.layers[0]["mlp_fc"] = torch.as_strided(w, w.shape, (1, w.shape[0]))  # the same address
+    assert m._fused() is None
+    m.layers[0]["mlp_fc"] = w
+    assert m._fused() is not None
