@@ -109,7 +109,7 @@ __device__ __forceinline__ void coeff_peak(const scope_coeff_params& p, const vo
 // (about 0.4 TB/s of its bytes with the library's forms), so the three
 // functions here leave out what their arguments never need.  Errors against
 // fp64 over 4 M arguments, library's in brackets: sin and cos 1.7e-8 rms (1.8e-8),
-// 7.0e-8 at most (7.2e-8); exp2 of a reduced argument is the library's own form.
+// 7.0e-8 at most (7.2e-8).
 //
 // sin and cos of |x| < kSincosMax: x - n·π/2 in two steps (n·1.57079637 fits
 // 41 bits and cancels exactly in the fma), Taylor polynomials on [-π/4, π/4]
@@ -138,7 +138,8 @@ __device__ __forceinline__ void coeff_sincos(float x, bool slow, float& s, float
   else sincos_reduced(x, s, c);
 }
 
-// e^-x of a finite x >= 0
+// e^-x of a finite x >= 0 as 2^(-x log2 e): log2 e as the sum of two floats, the
+// first product's rounding error carried by an fma, the integer part to the exponent
 __device__ __forceinline__ float exp_neg(float x) {
   const float t = x * -1.44269502f;  // -log2 e, and its remainder below
   const float lo = fmaf(x, -1.92596303e-8f, fmaf(x, -1.44269502f, -t));
