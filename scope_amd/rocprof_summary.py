@@ -34,7 +34,7 @@ KERNELS = ("attn_fwd_kernel", "attn_fwd_kernel(lse)", "attn_fwd_kernel(mass)", "
            "swa_rows_kernel", "swa_pad_kernel", "coeff_fwd_kernel", "coeff_bwd_kernel", "coeff_reg_kernel",
            "probe_mfma_kernel", "probe_copy_kernel")
 COPY = "copyBuffer"
-FWD_KINDS = {"0": "", "1": "(lse)", "2": "(mass)"}
+FWD_KINDS = {"0": "", "1": "(lse)", "2": "(mass)", "3": "(entry sums)"}
 
 
 def _base(name: str) -> str:
