@@ -72,7 +72,7 @@ class _Operator:
         _LIB.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
         _LIB.impl(name, torch._disable_dynamo(fn), "CompositeExplicitAutograd")
         self._op = getattr(getattr(torch.ops, _NS), name).default
-        self._setup = self._backward = self._function = None
+        self._recorded = None  # the autograd node class, with a backward formula
         _LIB.impl(name, self._autograd, "Autograd")
         self.__doc__ = fn.__doc__
 
@@ -83,41 +83,47 @@ class _Operator:
         torch.library.register_fake(f"{_NS}::{self._name}", fn, lib=_LIB)
         return fn
 
-    def register_autograd(self, backward, *, setup_context):
-        """``setup_context(ctx, inputs, output)`` and ``backward(ctx, *grads)``
+    def register_autograd(self, formula, *, setup_context):
+        """``setup_context(ctx, inputs, output)`` and ``formula(ctx, *grads)``
         as in ``torch.library.register_autograd``."""
-        self._backward, self._setup = backward, setup_context
+        run = self._run
 
-    def _make_function(self):
-        op, name, setup, formula = self._op, self._name, self._setup, self._backward
+        class Recorded(torch.autograd.Function):
+            @staticmethod
+            def forward(ctx, *inputs):
+                output = run(inputs)
+                setup_context(ctx, inputs, output)
+                return output
 
-        def forward(ctx, *args):
-            args = args if formula is not None else args[0]
-            with torch._C._AutoDispatchBelowAutograd():
-                out = op(*args)
-            if setup is not None:
-                setup(ctx, args, out)
-            return out
+            backward = staticmethod(formula)
 
-        def backward(ctx, *grads):
-            if formula is None:
-                raise RuntimeError(f"Trying to backward through {_NS}::{name} but no autograd formula was registered.")
-            return formula(ctx, *grads)
+        self._recorded = Recorded
 
-        return type(f"Scope_{name}", (torch.autograd.Function,),
-                    dict(forward=staticmethod(forward), backward=staticmethod(backward)))
-
-    def _autograd(self, *args):
-        if torch.is_grad_enabled():
-            tensors = [a for a in args if isinstance(a, Tensor)]
-            tensors += [b for a in args if isinstance(a, (list, tuple)) for b in a if isinstance(b, Tensor)]
-            if any(t.requires_grad for t in tensors):
-                if self._function is None:
-                    self._function = self._make_function()
-                # without a formula the tensors (a list's among them) only mark the outputs as not differentiable
-                return self._function.apply(*args) if self._backward is not None else self._function.apply(args, *tensors)
+    def _run(self, inputs):
+        """The operator below the autograd key."""
         with torch._C._AutoDispatchBelowAutograd():
-            return self._op(*args)
+            return self._op(*inputs)
+
+    def _autograd(self, *inputs):
+        # (tensors inside a list argument are constants, as custom_op takes them)
+        wanted = [x for x in inputs if isinstance(x, Tensor) and x.requires_grad] if torch.is_grad_enabled() else ()
+        if not wanted:
+            return self._run(inputs)
+        return self._recorded.apply(*inputs) if self._recorded else _NoGradient.apply(self, inputs, *wanted)
+
+
+class _NoGradient(torch.autograd.Function):
+    """Node of an operator that has no backward: a gradient that reaches one
+    of its results is an error, not a silent zero."""
+
+    @staticmethod
+    def forward(ctx, operator, inputs, *wanted):
+        ctx.operator = operator
+        return operator._run(inputs)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise RuntimeError(f"torch.ops.{_NS}.{ctx.operator._name} is not differentiable: detach its inputs or its results")
 
 
 def _operator(name):
