@@ -291,7 +291,10 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
     a.tokens[t] = tok;
     a.docs[t] = (t > 0 ? a.docs[t - 1] : 0) + (tok == p.eot ? 1 : 0);
   }
-  const int32_t doc_t = ok ? (t > 0 ? a.docs[t - 1] : 0) + (tok == p.eot ? 1 : 0) : 0;
+  // a token outside the vocabulary leaves docs[t] as it is and attends to that document
+  const int32_t doc_t = ok    ? (t > 0 ? a.docs[t - 1] : 0) + (tok == p.eot ? 1 : 0)
+                        : t >= 0 && t < p.T_cap ? a.docs[t]
+                                                : 0;
 
   Rows<2> wqkv, wfc;  // qkv rows wave and, below wave 4, wave + 8 of the workgroup's twelve
   Rows<1> wproj;      // wavefronts 0-3

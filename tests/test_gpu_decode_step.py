@@ -130,3 +130,23 @@ def test_replaced_weights_of_another_layout():
     assert m._fused() is None
     m.layers[0]["mlp_fc"] = w
     assert m._fused() is not None
+
+
+def test_token_outside_the_vocabulary_stays_in_its_document():
+    """After documents have opened, such a token (the padded columns of the
+    logits have ids past the vocabulary) attends to the document its position
+    carries, as in the layer-by-layer step, and its k and v rows, which later
+    tokens read, are the same."""
+    one, ref = (_model(384, f, 6, use_graph=False) for f in (True, False))
+    toks = torch.randint(0, 50256, (140,), generator=torch.Generator().manual_seed(4))
+    toks[[40, 100]] = 50256
+    bad = torch.tensor([50280], device=DEV)
+    for m in (one, ref):
+        m.prefill(toks[:128])
+        m.step(toks[128])
+    for s in range(129, 135):
+        tok = bad if s == 131 else toks[s]
+        a, b = one.step(tok), ref.step(tok)
+        assert (a - b).abs().max().item() <= 5e-2, f"position {s}"
+    assert torch.equal(one.docs, ref.docs)
+    _close(one, ref, 135)
