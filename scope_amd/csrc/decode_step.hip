@@ -195,6 +195,8 @@ __device__ __forceinline__ float rf_bf16(float x) { return __uint_as_float(pk_bf
 __device__ __forceinline__ float lo_f(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float hi_f(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 
+__device__ __forceinline__ float relu_nan(float x) { return x < 0.f ? 0.f : x; }  // keeps a NaN
+
 // acc += the product of eight bf16 weights and eight inputs
 __device__ __forceinline__ float dot8(const uint4& w, const float* x, float acc) {
   const uint32_t q[4] = {w.x, w.y, w.z, w.w};
@@ -231,7 +233,8 @@ struct Rows {
 };
 
 // Merge of eight wavefronts' (o, m, l) at features lane and lane + 64:
-// log2-domain maxima, entries without a key have m = -inf.
+// log2-domain maxima, entries without a key have m = -inf and l = 0.  A NaN
+// in l stays, here and in the merges after it, whatever its m.
 struct Merged {
   float M, L, O0, O1;
 };
@@ -242,7 +245,7 @@ __device__ __forceinline__ Merged merge_waves(const float (&o)[kCW][kHd], const 
   for (int w = 0; w < kCW; ++w) r.M = fmaxf(r.M, m[w]);
 #pragma unroll
   for (int w = 0; w < kCW; ++w) {
-    if (m[w] == -INFINITY) continue;
+    if (m[w] == -INFINITY && l[w] == 0.f) continue;
     const float s = __builtin_amdgcn_exp2f(m[w] - r.M);
     r.L = fmaf(l[w], s, r.L);
     r.O0 = fmaf(o[w][lane], s, r.O0);
@@ -467,6 +470,8 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
           }
           m = fmaxf(m, __shfl_xor(m, 16, kWave));
           m = fmaxf(m, __shfl_xor(m, 32, kWave));
+          // fmaxf skips NaN scores: with nothing but them, any offset keeps them in l and o
+          if (m == -INFINITY && __any(s[0] != s[0] || s[1] != s[1] || s[2] != s[2] || s[3] != s[3])) m = 0.f;
           if (m != -INFINITY) {  // wavefront-uniform
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
@@ -513,7 +518,7 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
             const uint64_t* const q[4] = {pe + lane, pe + lane + 64, pe + kHd, pe + kHd + 1};
             float f[4];
             poll_f32<4>(q, seq, f, wt);
-            if (f[2] == -INFINITY) continue;
+            if (f[2] == -INFINITY && f[3] == 0.f) continue;
             const float Mn = fmaxf(r.M, f[2]);
             const float sa = r.M == Mn ? 1.f : __builtin_amdgcn_exp2f(r.M - Mn), sb = __builtin_amdgcn_exp2f(f[2] - Mn);
             r = Merged{Mn, fmaf(f[3], sb, r.L * sa), fmaf(f[0], sb, r.O0 * sa), fmaf(f[1], sb, r.O1 * sa)};
@@ -523,10 +528,10 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
           __syncthreads();  // the merged entries
           if (wave == 0) {
             const Merged y = merge_waves(sh.o[1], sh.m[1], sh.l[1], lane);
-            const float inv = y.L > 0.f ? 1.f / y.L : 0.f;
+            const float inv = 1.f / y.L;  // (L = 0: no key)
             uint32_t* py = lv + kYOff + head * kHd + lane;
-            publish(py, r_bf16(y.L > 0.f ? y.O0 * inv : 0.f), tag);
-            publish(py + 64, r_bf16(y.L > 0.f ? y.O1 * inv : 0.f), tag);
+            publish(py, r_bf16(y.L == 0.f ? 0.f : y.O0 * inv), tag);
+            publish(py + 64, r_bf16(y.L == 0.f ? 0.f : y.O1 * inv), tag);
           }
         }
       }
@@ -546,7 +551,7 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
     }
     // ---- MLP
     {
-      const float h0 = fmaxf(wfc.run(0, x), 0.f), h1 = fmaxf(wfc.run(1, x), 0.f);
+      const float h0 = relu_nan(wfc.run(0, x)), h1 = relu_nan(wfc.run(1, x));
       if (lane == 0) {
         sh.rows[pr][2 * wave] = r_bf16(__fmul_rn(h0, h0));
         sh.rows[pr][2 * wave + 1] = r_bf16(__fmul_rn(h1, h1));

@@ -150,3 +150,22 @@ def test_token_outside_the_vocabulary_stays_in_its_document():
         assert (a - b).abs().max().item() <= 5e-2, f"position {s}"
     assert torch.equal(one.docs, ref.docs)
     _close(one, ref, 135)
+
+
+@pytest.mark.parametrize("where", ["query", "hidden", "key", "value"])
+def test_nan_reaches_the_logits(where):
+    """A NaN inside a layer (an expired wait goes on with one) is in every
+    logit: a head's whole query (all scores NaN), one hidden unit of the MLP,
+    one visible key or value (some scores or products NaN)."""
+    m = _model(256, True, 6, use_graph=False)
+    toks = torch.randint(0, 50256, (140,), generator=torch.Generator().manual_seed(6))
+    m.prefill(toks[:128])
+    m.step(toks[128])
+    assert bool(torch.isfinite(m.step(toks[129])).all())
+    if where == "query":
+        m.layers[2]["qkv"][128:256] = float("nan")  # head 1
+    elif where == "hidden":
+        m.layers[2]["mlp_fc"][77] = float("nan")
+    else:
+        (m.k_cache if where == "key" else m.v_cache)[2][1, 60] = float("nan")
+    assert bool(torch.isnan(m.step(toks[130])).all())
