@@ -109,14 +109,21 @@ __device__ __forceinline__ float row_sum16(float x) {
 
 // a wavefront's waits: when one lasts longer than the limit, it and all later ones end at once with NaN
 struct StepWait {
-  uint64_t t0, limit;
+  uint64_t limit;
   uint32_t* status;
   int32_t* host_status;
   bool dead;
 };
 
-__device__ __forceinline__ bool step_expired(StepWait& w, int it) {
-  if (!w.dead && (it & 63) == 63 && static_cast<uint64_t>(wall_clock64()) - w.t0 > w.limit) {
+// Poll `it` of a wait found nothing: whether the wait ends.  The time counts from
+// the wait's 64th poll (t0), not from the kernel's start: a kernel that was held
+// up between its waits has not waited.
+__device__ __forceinline__ bool step_expired(StepWait& w, int it, uint64_t& t0) {
+  if (w.dead || (it & 63) != 63) return w.dead;
+  const uint64_t now = static_cast<uint64_t>(wall_clock64());
+  if (it == 63) {
+    t0 = now;
+  } else if (now - t0 > w.limit) {
     w.dead = true;
     __hip_atomic_store(w.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (w.host_status) __hip_atomic_store(w.host_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -128,6 +135,7 @@ __device__ __forceinline__ bool step_expired(StepWait& w, int it) {
 template <int N>
 __device__ __forceinline__ void poll_bf16(const uint64_t* p, int stride, uint32_t tag, uint64_t (&v)[N], StepWait& w) {
   const uint64_t want = (static_cast<uint64_t>(tag) << 48) | (static_cast<uint64_t>(tag) << 16);
+  uint64_t t0 = 0;
   for (int it = 0;; ++it) {
 #pragma unroll
     for (int j = 0; j < N; ++j)
@@ -136,7 +144,7 @@ __device__ __forceinline__ void poll_bf16(const uint64_t* p, int stride, uint32_
 #pragma unroll
     for (int j = 0; j < N; ++j) diff |= (v[j] ^ want) & 0xffff0000ffff0000ull;
     if (__all(diff == 0)) return;
-    if (step_expired(w, it)) break;
+    if (step_expired(w, it, t0)) break;
   }
 #pragma unroll
   for (int j = 0; j < N; ++j) v[j] = kNanBf16 | (static_cast<uint64_t>(kNanBf16) << 32);
@@ -145,6 +153,7 @@ __device__ __forceinline__ void poll_bf16(const uint64_t* p, int stride, uint32_
 // N tagged fp32 words of this lane at q[j]
 template <int N>
 __device__ __forceinline__ void poll_f32(const uint64_t* const (&q)[N], uint32_t seq, float (&f)[N], StepWait& w) {
+  uint64_t t0 = 0;
   for (int it = 0;; ++it) {
     uint64_t v[N];
     uint32_t diff = 0;
@@ -156,7 +165,7 @@ __device__ __forceinline__ void poll_f32(const uint64_t* const (&q)[N], uint32_t
       f[j] = __uint_as_float(static_cast<uint32_t>(v[j]));
     }
     if (__all(diff == 0)) return;
-    if (step_expired(w, it)) break;
+    if (step_expired(w, it, t0)) break;
   }
 #pragma unroll
   for (int j = 0; j < N; ++j) f[j] = __builtin_nanf("");
@@ -256,14 +265,15 @@ __device__ __forceinline__ Merged merge_waves(const float (&o)[kCW][kHd], const 
 
 __global__ __launch_bounds__(64) void step_lock_kernel(uint32_t* work, int32_t* host_status, uint64_t limit) {
   if (threadIdx.x != 0) return;
-  StepWait w{static_cast<uint64_t>(wall_clock64()), limit, work + 1, host_status, __hip_atomic_load(work + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0};
+  StepWait w{limit, work + 1, host_status, __hip_atomic_load(work + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0};
   // with the status set the step takes no lock and its kernel releases none
+  uint64_t t0 = 0;
   for (int it = 0; !w.dead; ++it) {
     int free_ = 0;
     if (__hip_atomic_compare_exchange_strong(&g_step_lock, &free_, 1, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT))
       return;
-    if (step_expired(w, it)) return;
+    if (step_expired(w, it, t0)) return;
     __builtin_amdgcn_s_sleep(8);
   }
 }
@@ -276,7 +286,7 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
   // (atomic loads: workgroup 0 writes the counter and the position at its end)
   const uint32_t seq = __hip_atomic_load(a.work, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1, tag = seq & 0xffffu;
   const bool dead0 = __hip_atomic_load(a.work + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-  StepWait wt{static_cast<uint64_t>(wall_clock64()), p.spin_ticks, a.work + 1, a.host_status, dead0};
+  StepWait wt{p.spin_ticks, a.work + 1, a.host_status, dead0};
   const int64_t tok = *a.tok, t = __hip_atomic_load(a.t_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const bool ok = tok >= 0 && tok < p.vocab && t >= 0 && t < p.T_cap;
   const bool pos_ok = t >= 0 && t < p.T_cap && t < p.rot_rows;
