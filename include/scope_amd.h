@@ -603,7 +603,9 @@ int scope_decoder_add_norm(int64_t T, int dm, float eps, const uint16_t* x, cons
  * q-block: the lists of layer.kv_num / kv_idx are those of t's block): what
  * scope_decoder_step_prologue, then per layer scope_decoder_gemv (qkv),
  * scope_decode_attn_glue_at and scope_decoder_gemv (projection, MLP) compute,
- * in one launch of resident workgroups.  tokens[t], docs[t] and cache rows t
+ * in one launch of workgroups that wait for each other.  It runs on those that
+ * are on the device when one of them has waited gang_ticks (100 MHz) for the
+ * rest, and so ends beside any other kernels.  tokens[t], docs[t] and cache rows t
  * are written, x_out [dm] gets the last layer's output, *t_dev becomes t + 1.
  * The layers' lambdas are (1, 0), the U-net skips' weights 1.
  *   layers      device array of p->layers records (qkv NULL: no attention;
@@ -614,7 +616,7 @@ int scope_decoder_add_norm(int64_t T, int dm, float eps, const uint16_t* x, cons
  *               than spin_ticks (100 MHz); the step then gives NaN)
  *   host_status pinned host int that also gets the status, or NULL
  * scope_decoder_step_supported: whether the shape is served and the current
- * device holds all workgroups at once. */
+ * device, when idle, holds all workgroups at once. */
 typedef struct {
   const uint16_t* qkv;      /* [3·H·D][dm] */
   const uint16_t* proj;     /* [dm][H·D] */
@@ -631,9 +633,10 @@ typedef struct {
 
 typedef struct {
   int layers, H, D, dm, mlp, bs, maxkv;
+  int workgroups; /* launched: 1 .. 256, 0 for 256 (fewer wait gang_ticks and are slower) */
   float scale, eps;
   int64_t T_cap, vocab, eot, rot_rows, rot_st, k_sh, k_st, v_sh, v_st;
-  uint64_t spin_ticks;
+  uint64_t spin_ticks, gang_ticks;
 } scope_decoder_step_params;
 
 int scope_decoder_step_supported(const scope_decoder_step_params* p);

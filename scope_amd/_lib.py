@@ -88,9 +88,9 @@ class DecoderLayer(C.Structure):
 
 class DecoderStepParams(C.Structure):
     _fields_ = [("layers", c_int), ("H", c_int), ("D", c_int), ("dm", c_int), ("mlp", c_int), ("bs", c_int),
-                ("maxkv", c_int), ("scale", c_float), ("eps", c_float), ("T_cap", c_int64), ("vocab", c_int64),
-                ("eot", c_int64), ("rot_rows", c_int64), ("rot_st", c_int64), ("k_sh", c_int64), ("k_st", c_int64),
-                ("v_sh", c_int64), ("v_st", c_int64), ("spin_ticks", c_uint64)]
+                ("maxkv", c_int), ("workgroups", c_int), ("scale", c_float), ("eps", c_float), ("T_cap", c_int64),
+                ("vocab", c_int64), ("eot", c_int64), ("rot_rows", c_int64), ("rot_st", c_int64), ("k_sh", c_int64), ("k_st", c_int64),
+                ("v_sh", c_int64), ("v_st", c_int64), ("spin_ticks", c_uint64), ("gang_ticks", c_uint64)]
 
 
 P = c_void_p

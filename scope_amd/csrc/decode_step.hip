@@ -31,16 +31,22 @@
 // Rows published by the wavefronts one by one, not as one store per workgroup,
 // took 0.40 ms: each was a write of its own to the same memory line.
 //
-// All workgroups must be resident together.  The launch is refused where the
-// device cannot hold them, and a lock in device memory, taken by a
-// one-wavefront launch before and released at the end, lets one such kernel
-// of the process run at a time (two half-resident ones would wait for each
-// other).  Every wait ends: after spin_ticks the waiter sets the status word
+// The workgroups of a step wait for each other, so only workgroups that are
+// there may take part: each adds itself to a counter as it starts, and the step
+// begins when all 256 have, or when one has waited gang_ticks for the rest and
+// closes the counter: those that are there then share all the work (the same
+// sums in the same order, the weights loaded as they are used), later ones
+// leave at once.  So a step ends whatever else holds the device: kernels of
+// other streams, another process's step that got the other half of the chip.
+// (Without it two processes whose steps started together, each half-resident,
+// waited for each other.)  Within a process a lock in device memory, taken by a
+// one-wavefront launch before, lets one step run at a time; a lock that is not
+// free within 2 ms is not waited for any longer.
+// Every other wait ends too: after spin_ticks the waiter sets the status word
 // and goes on with NaN, which reaches every row through the tagged words.
-// The lock does not reach other processes: two that step on one device at the
-// same moment may wait for each other until that limit (capacity for two such
-// kernels, 128 registers a lane, spills 93 of the 181).
 #include <math.h>
+
+#include <mutex>
 
 #include "common.h"
 
@@ -56,8 +62,12 @@ constexpr int kMaxKv = 32;           // list entries per head
 constexpr float kStepLog2e = 1.4426950408889634f;
 constexpr uint32_t kNanBf16 = 0x7fc0u;
 
-// workspace: 64 words of header (0: steps done, 1: status), then per layer the tagged vectors
+// workspace: 64 words of header (0: steps done, 1: status, 2: the step's workgroups,
+// 3: whether the step holds the lock), then per layer the tagged vectors
 constexpr int64_t kHeadWords = 64;
+constexpr int kGangWord = 2, kLockWord = 3;
+constexpr uint32_t kClosed = 0x80000000u;
+constexpr uint64_t kLockTicks = 200000;  // 2 ms: what six steps take
 constexpr int64_t kQkvOff = 0, kYOff = kQkvOff + 3 * kDm, kX1Off = kYOff + kDm, kHOff = kX1Off + kDm,
                   kX2Off = kHOff + kMlp, kPartOff = kX2Off + kDm;  // 32-bit words
 constexpr int kPartWords = (kHd + 2) * 2;                          // one entry's o, m, l as 64-bit words
@@ -184,13 +194,15 @@ __device__ __forceinline__ void publish_f32(uint64_t* p, float x, uint32_t seq) 
 struct StepShared {
   __attribute__((aligned(16))) uint16_t xs[2][kDm];  // the phase's input, two phases alternating
   float ss[2][kCW];                                  // the wavefronts' sums of squares
-  float part[2][4][kCW];                             // MLP output: (row, segment) sums, two layers alternating
+  float part[2][4][kCW];                             // MLP output: (row, segment) sums, two parts alternating
   uint32_t rows[2][16];                              // output words to publish, two phases alternating
   uint16_t xraw[2][kDm];                             // the residual stream before the attention and before the MLP
   uint16_t skip[kMaxSkip][kDm];                      // layer outputs for the U-net skips (each lane its own features)
   float gq[kHd];                                     // attention: the rotated query, and the token's k and v rows
   __attribute__((aligned(16))) uint16_t gk[kHd], gv[kHd];
   float o[2][kCW][kHd], m[2][kCW], l[2][kCW];        // the wavefronts' attention sums and their merged entries
+  int gang;                                          // the step's workgroups
+  uint32_t rank;                                     // the gang word as this workgroup's arrival found it
 };
 
 __device__ __forceinline__ uint32_t pk_bf16(float lo, float hi) {  // round to nearest even
@@ -263,24 +275,79 @@ __device__ __forceinline__ Merged merge_waves(const float (&o)[kCW][kHd], const 
   return r;
 }
 
-__global__ __launch_bounds__(64) void step_lock_kernel(uint32_t* work, int32_t* host_status, uint64_t limit) {
+__device__ __forceinline__ int step_next_att(const StepArgs& a, int i) {  // layer i or the next one with attention
+  while (i < a.p.layers && !a.layers[i].qkv) ++i;
+  return i;
+}
+
+// Before a step: the gang word is cleared, and the process's step lock taken, or
+// not within kLockTicks (whether it was is kept for the release).
+__global__ __launch_bounds__(64) void step_begin_kernel(uint32_t* work) {
   if (threadIdx.x != 0) return;
-  StepWait w{limit, work + 1, host_status, __hip_atomic_load(work + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0};
-  // with the status set the step takes no lock and its kernel releases none
-  uint64_t t0 = 0;
-  for (int it = 0; !w.dead; ++it) {
+  __hip_atomic_store(work + kGangWord, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t t0 = static_cast<uint64_t>(wall_clock64());
+  uint32_t took = 0;
+  do {
     int free_ = 0;
-    if (__hip_atomic_compare_exchange_strong(&g_step_lock, &free_, 1, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
+    took = __hip_atomic_compare_exchange_strong(&g_step_lock, &free_, 1, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+    if (!took) __builtin_amdgcn_s_sleep(8);
+  } while (!took && static_cast<uint64_t>(wall_clock64()) - t0 < kLockTicks);
+  __hip_atomic_store(work + kLockWord, took, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The number of workgroups a step runs on, for one of them.  Each adds itself to
+// the gang word as it starts: arrivals in the low 16 bits, and once it is closed
+// kClosed and the size at that moment in bits 16-30.  Ends when all kG have
+// arrived or when a workgroup that waited longer than the limit closes the gang
+// with those that are there; a closing and a full gang exclude each other (the
+// compare-and-swap expects fewer arrivals).
+__device__ __forceinline__ int step_gang(uint32_t* word, uint64_t limit) {
+  uint64_t t0 = 0;
+  for (bool first = true;; first = false) {
+    uint32_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (w & kClosed) return static_cast<int>((w & ~kClosed) >> 16);
+    if (w == kG) return kG;
+    const uint64_t now = static_cast<uint64_t>(wall_clock64());
+    if (first) t0 = now;
+    if (now - t0 >= limit &&
+        __hip_atomic_compare_exchange_strong(word, &w, kClosed | (w << 16) | w, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT))
-      return;
-    if (step_expired(w, it, t0)) return;
-    __builtin_amdgcn_s_sleep(8);
+      return static_cast<int>(w);
   }
 }
 
-__global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
-  __shared__ StepShared sh;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wg = blockIdx.x;
+// the weights a workgroup holds in registers: rows of part v of every product
+struct StepWeights {
+  Rows<2> qkv, fc;  // qkv rows wave and, below wave 4, wave + 8 of the part's twelve
+  Rows<1> proj;     // wavefronts 0-3
+  uint4 mp[4];      // MLP output: segment `wave` of the four rows
+  __device__ __forceinline__ void load_qkv(const scope_decoder_layer& l, int v, int wave, int lane) {
+    qkv.load(l.qkv, 12 * v + wave, wave < 4 ? 8 : 0, lane);
+  }
+  __device__ __forceinline__ void load_proj(const scope_decoder_layer& l, int v, int wave, int lane) {
+    proj.load(l.proj, 4 * v + (wave & 3), 0, lane);
+  }
+  __device__ __forceinline__ void load_fc(const scope_decoder_layer& l, int v, int wave, int lane) {
+    fc.load(l.mlp_fc, 16 * v + 2 * wave, 1, lane);
+  }
+  __device__ __forceinline__ void load_mp(const scope_decoder_layer& l, int v, int wave, int lane) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      mp[j] = *reinterpret_cast<const uint4*>(l.mlp_proj + static_cast<int64_t>(4 * v + j) * kMlp + wave * 512 + 8 * lane);
+  }
+};
+
+// The step on n workgroups, of which this is number wg.  FULL: n = kG, part wg
+// is this workgroup's, its weights in registers a layer ahead; whether all are
+// there is looked at after its first rows are published, when the answer is
+// ready: false if not, before anything but those rows (which are the same on any
+// number of workgroups) is written.  Otherwise each workgroup takes the parts
+// wg, wg + n, .. of every phase, weights loaded as they are used: the same sums
+// in the same order.
+template <bool FULL>
+__device__ __forceinline__ bool step_run(const StepArgs& a, StepShared& sh, StepWeights& W, const int wg, const int n) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const scope_decoder_step_params& p = a.p;
   const int L = p.layers, nskip = L / 2, maxkv = p.maxkv;
   // (atomic loads: workgroup 0 writes the counter and the position at its end)
@@ -292,45 +359,21 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
   const bool pos_ok = t >= 0 && t < p.T_cap && t < p.rot_rows;
   uint32_t* const vec = a.work + kHeadWords;
   const int64_t lw = step_layer_words(maxkv);
-  // this workgroup's (head, list entry), if it has one
-  const int ntask = kHeads * maxkv, every = kG / ntask;
-  const bool att = wg % every == 0 && wg / every < ntask;
-  const int task = wg / every, head = att ? task / maxkv : 0, ent = att ? task % maxkv : 0;
-  auto next_att = [&](int i) {  // the next layer with attention (L: none)
-    while (i < L && !a.layers[i].qkv) ++i;
-    return i;
-  };
-  if (wg == 0 && tid == 0 && ok) {
-    a.tokens[t] = tok;
-    a.docs[t] = (t > 0 ? a.docs[t - 1] : 0) + (tok == p.eot ? 1 : 0);
-  }
+  const int ntask = kHeads * maxkv, every = kG / ntask;  // tasks: (head, list entry), the entries of a head in a row
   // a token outside the vocabulary leaves docs[t] as it is and attends to that document
   const int32_t doc_t = ok    ? (t > 0 ? a.docs[t - 1] : 0) + (tok == p.eot ? 1 : 0)
                         : t >= 0 && t < p.T_cap ? a.docs[t]
                                                 : 0;
-
-  Rows<2> wqkv, wfc;  // qkv rows wave and, below wave 4, wave + 8 of the workgroup's twelve
-  Rows<1> wproj;      // wavefronts 0-3
-  uint4 wmp[4];       // MLP output: segment `wave` of the four rows
-  auto load_qkv = [&](int i) { wqkv.load(a.layers[i].qkv, 12 * wg + wave, wave < 4 ? 8 : 0, lane); };
-  auto load_proj = [&](int i) { wproj.load(a.layers[i].proj, 4 * wg + (wave & 3), 0, lane); };
-  auto load_fc = [&](int i) { wfc.load(a.layers[i].mlp_fc, 16 * wg + 2 * wave, 1, lane); };
-  auto load_mp = [&](int i) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      wmp[j] = *reinterpret_cast<const uint4*>(a.layers[i].mlp_proj + static_cast<int64_t>(4 * wg + j) * kMlp + wave * 512 +
-                                               8 * lane);
+  auto parts_of = [&](auto&& f) {  // f(v) for this workgroup's parts of a product
+    if constexpr (FULL) {
+      f(wg);
+    } else {
+      for (int v = wg; v < kG; v += n) f(v);
+    }
   };
-  const int i0 = next_att(0);
-  if (i0 < L) {
-    load_qkv(i0);
-    load_proj(i0);
-  }
-  load_fc(0);
-  load_mp(0);
 
   const int sub = lane >> 4, ch = lane & 15, f0 = 128 * wave + 2 * lane;  // f0: this lane's two features of a vector
-  int pb = 0;
+  int pb = 0, pp = 0;  // which of the two buffers: xs and ss, part
   float x0, x1;   // features f0, f0 + 1
   float x[16];    // inputs of whole rows: columns 8·lane.. of both halves
   auto poll_x = [&](const uint32_t* src) {
@@ -366,6 +409,11 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
     pb ^= 1;
   };
 
+  auto all_there = [&]() {
+    if (tid == 0) sh.gang = step_gang(a.work + kGangWord, p.gang_ticks);
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(sh.gang) == kG;
+  };
   for (int i = 0; i < L; ++i) {
     const scope_decoder_layer lay = a.layers[i];
     uint32_t* const lv = vec + i * lw;
@@ -391,23 +439,26 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
     spread(rms());
     int res = 0;
     if (lay.qkv) {
-      const int nx = next_att(i + 1);
+      const int nx = FULL ? step_next_att(a, i + 1) : L;
       // ---- qkv
-      {
-        const float z0 = wqkv.run(0, x), z1 = wqkv.run(1, x);
+      parts_of([&](int v) {
+        if (!FULL) W.load_qkv(lay, v, wave, lane);
+        const float z0 = W.qkv.run(0, x), z1 = W.qkv.run(1, x);
         if (lane == 0) {
           sh.rows[pr][wave] = r_bf16(z0);
           if (wave < 4) sh.rows[pr][wave + 8] = r_bf16(z1);
         }
-        publish_rows(lv + kQkvOff + 12 * wg, 12);
-      }
-      if (nx < L) load_qkv(nx);
+        publish_rows(lv + kQkvOff + 12 * v, 12);
+      });
+      if (FULL && i == 0 && !all_there()) return false;
+      if (nx < L) W.load_qkv(a.layers[nx], wg, wave, lane);
       // ---- attention: one (head, list entry)
-      if (att) {
+      uint64_t* const parts = reinterpret_cast<uint64_t*>(lv + kPartOff);
+      auto attend = [&](int task) __attribute__((always_inline)) {
+        const int head = task / maxkv, ent = task % maxkv;
         // keys 16·wave .. +15 of the entry's block: sixteen lanes per row, four
         // rows at a time; the rows are loaded while the qkv vector is on its way
-        const int n = lay.kv_num[head];
-        const int64_t kblk = ent < n ? lay.kv_idx[static_cast<int64_t>(head) * maxkv + ent] : -1;
+        const int64_t kblk = ent < lay.kv_num[head] ? lay.kv_idx[static_cast<int64_t>(head) * maxkv + ent] : -1;
         const int64_t k0 = kblk * kBs;
         const bool use = kblk >= 0 && k0 <= t && k0 + kBs <= p.T_cap && pos_ok;
         uint4 ku[4], vu[4];
@@ -420,7 +471,7 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
             const int64_t j = k0 + 16 * wave + 4 * it + sub;
             ku[it] = *reinterpret_cast<const uint4*>(kr + j * p.k_st);
             vu[it] = *reinterpret_cast<const uint4*>(vr + j * p.v_st);
-            dj[it] = j < t ? a.docs[j] : doc_t;  // docs[t] is being written by workgroup 0
+            dj[it] = j < t ? a.docs[j] : doc_t;  // docs[t] is written at the end
           }
         }
         // the token's q (wavefront 0), k (1) and v (2) of the head: lane l holds features 2l and 2l + 1
@@ -510,7 +561,6 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
         }
         if (lane == 0) sh.m[0][wave] = m, sh.l[0][wave] = l;
         __syncthreads();  // the wavefronts' sums
-        uint64_t* const parts = reinterpret_cast<uint64_t*>(lv + kPartOff);
         if (wave == 0) {
           const Merged r = merge_waves(sh.o[0], sh.m[0], sh.l[0], lane);
           uint64_t* pp = parts + static_cast<int64_t>(task) * (kHd + 2);
@@ -521,53 +571,72 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
             publish_f32(pp + kHd + 1, r.L, seq);
           }
         }
-        if (ent == 0) {  // this workgroup merges the head's entries, wavefront w the entries w, w + 8, ..
-          Merged r{-INFINITY, 0.f, 0.f, 0.f};
-          for (int e = wave; e < maxkv; e += kCW) {
-            const uint64_t* pe = parts + (static_cast<int64_t>(head) * maxkv + e) * (kHd + 2);
-            const uint64_t* const q[4] = {pe + lane, pe + lane + 64, pe + kHd, pe + kHd + 1};
-            float f[4];
-            poll_f32<4>(q, seq, f, wt);
-            if (f[2] == -INFINITY && f[3] == 0.f) continue;
-            const float Mn = fmaxf(r.M, f[2]);
-            const float sa = r.M == Mn ? 1.f : __builtin_amdgcn_exp2f(r.M - Mn), sb = __builtin_amdgcn_exp2f(f[2] - Mn);
-            r = Merged{Mn, fmaf(f[3], sb, r.L * sa), fmaf(f[0], sb, r.O0 * sa), fmaf(f[1], sb, r.O1 * sa)};
-          }
-          sh.o[1][wave][lane] = r.O0, sh.o[1][wave][lane + 64] = r.O1;
-          if (lane == 0) sh.m[1][wave] = r.M, sh.l[1][wave] = r.L;
-          __syncthreads();  // the merged entries
-          if (wave == 0) {
-            const Merged y = merge_waves(sh.o[1], sh.m[1], sh.l[1], lane);
-            const float inv = 1.f / y.L;  // (L = 0: no key)
-            uint32_t* py = lv + kYOff + head * kHd + lane;
-            publish(py, r_bf16(y.L == 0.f ? 0.f : y.O0 * inv), tag);
-            publish(py + 64, r_bf16(y.L == 0.f ? 0.f : y.O1 * inv), tag);
-          }
+      };
+      // merges the head's entries, wavefront w the entries w, w + 8, ..
+      auto merge_head = [&](int head) __attribute__((always_inline)) {
+        Merged r{-INFINITY, 0.f, 0.f, 0.f};
+        for (int e = wave; e < maxkv; e += kCW) {
+          const uint64_t* pe = parts + (static_cast<int64_t>(head) * maxkv + e) * (kHd + 2);
+          const uint64_t* const q[4] = {pe + lane, pe + lane + 64, pe + kHd, pe + kHd + 1};
+          float f[4];
+          poll_f32<4>(q, seq, f, wt);
+          if (f[2] == -INFINITY && f[3] == 0.f) continue;
+          const float Mn = fmaxf(r.M, f[2]);
+          const float sa = r.M == Mn ? 1.f : __builtin_amdgcn_exp2f(r.M - Mn), sb = __builtin_amdgcn_exp2f(f[2] - Mn);
+          r = Merged{Mn, fmaf(f[3], sb, r.L * sa), fmaf(f[0], sb, r.O0 * sa), fmaf(f[1], sb, r.O1 * sa)};
+        }
+        sh.o[1][wave][lane] = r.O0, sh.o[1][wave][lane + 64] = r.O1;
+        if (lane == 0) sh.m[1][wave] = r.M, sh.l[1][wave] = r.L;
+        __syncthreads();  // the merged entries
+        if (wave == 0) {
+          const Merged y = merge_waves(sh.o[1], sh.m[1], sh.l[1], lane);
+          const float inv = 1.f / y.L;  // (L = 0: no key)
+          uint32_t* py = lv + kYOff + head * kHd + lane;
+          publish(py, r_bf16(y.L == 0.f ? 0.f : y.O0 * inv), tag);
+          publish(py + 64, r_bf16(y.L == 0.f ? 0.f : y.O1 * inv), tag);
+        }
+      };
+      if constexpr (FULL) {  // a task on every third workgroup or so
+        if (wg % every == 0 && wg / every < ntask) {
+          attend(wg / every);
+          if (wg / every % maxkv == 0) merge_head(wg / every / maxkv);
+        }
+      } else {  // (every entry of this workgroup's before it waits for another's)
+        for (int task = wg; task < ntask; task += n) attend(task);
+        for (int task = wg; task < ntask; task += n) {
+          if (task % maxkv) continue;
+          merge_head(task / maxkv);
+          __syncthreads();  // the merged entries are read
         }
       }
       // ---- output projection and residual
       poll_x(lv + kYOff);
       spread(1.f);
-      if (wave < 4) {
-        const float z = wproj.run(0, x);
-        if (lane == 0) sh.rows[pr][wave] = r_bf16(__fadd_rn(bf16_to_f32(sh.xraw[0][4 * wg + wave]), z));
-      }
-      publish_rows(lv + kX1Off + 4 * wg, 4);
-      if (nx < L) load_proj(nx);
+      parts_of([&](int v) {
+        if (!FULL) W.load_proj(lay, v, wave, lane);
+        if (wave < 4) {
+          const float z = W.proj.run(0, x);
+          if (lane == 0) sh.rows[pr][wave] = r_bf16(__fadd_rn(bf16_to_f32(sh.xraw[0][4 * v + wave]), z));
+        }
+        publish_rows(lv + kX1Off + 4 * v, 4);
+      });
+      if (nx < L) W.load_proj(a.layers[nx], wg, wave, lane);
       poll_x(lv + kX1Off);
       *reinterpret_cast<uint32_t*>(&sh.xraw[1][f0]) = pk_bf16(x0, x1);
       res = 1;
       spread(rms());
     }
     // ---- MLP
-    {
-      const float h0 = relu_nan(wfc.run(0, x)), h1 = relu_nan(wfc.run(1, x));
+    parts_of([&](int v) {
+      if (!FULL) W.load_fc(lay, v, wave, lane);
+      const float h0 = relu_nan(W.fc.run(0, x)), h1 = relu_nan(W.fc.run(1, x));
       if (lane == 0) {
         sh.rows[pr][2 * wave] = r_bf16(__fmul_rn(h0, h0));
         sh.rows[pr][2 * wave + 1] = r_bf16(__fmul_rn(h1, h1));
       }
-      publish_rows(lv + kHOff + 16 * wg, 16);
-    }
+      publish_rows(lv + kHOff + 16 * v, 16);
+    });
+    if (FULL && i == 0 && !lay.qkv && !all_there()) return false;
     {
       // this lane's eight inputs of segment `wave`, straight from the published words
       uint64_t v[4];
@@ -578,29 +647,63 @@ __global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
     // Loads return in order, so a poll also waits for every load before it: these
     // are issued after the poll.  (The MLP's weights a layer ahead but loaded
     // during the attention, and qkv's during the MLP: 350 instead of 314 us.)
-    if (i + 1 < L) load_fc(i + 1);
+    if (FULL && i + 1 < L) W.load_fc(a.layers[i + 1], wg, wave, lane);
+    parts_of([&](int v) {
+      if (!FULL) W.load_mp(lay, v, wave, lane);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float z = step_wave_sum(dot8(wmp[j], x, 0.f));
-      if (lane == 0) sh.part[i & 1][j][wave] = z;
-    }
-    if (i + 1 < L) load_mp(i + 1);
-    __syncthreads();  // MLP output sums
-    if (wave == 0 && lane < 4) {
-      float z = 0.f;
+      for (int j = 0; j < 4; ++j) {
+        const float z = step_wave_sum(dot8(W.mp[j], x, 0.f));
+        if (lane == 0) sh.part[pp][j][wave] = z;
+      }
+      if (FULL && i + 1 < L) W.load_mp(a.layers[i + 1], wg, wave, lane);
+      __syncthreads();  // MLP output sums
+      if (wave == 0 && lane < 4) {
+        float z = 0.f;
 #pragma unroll
-      for (int w = 0; w < kCW; ++w) z += sh.part[i & 1][lane][w];
-      const uint16_t y = r_bf16(__fadd_rn(bf16_to_f32(sh.xraw[res][4 * wg + lane]), rf_bf16(z)));
-      if (i + 1 < L) publish(lv + kX2Off + 4 * wg + lane, y, tag);
-      else a.x_out[4 * wg + lane] = wt.dead ? static_cast<uint16_t>(kNanBf16) : y;
-    }
+        for (int w = 0; w < kCW; ++w) z += sh.part[pp][lane][w];
+        const uint16_t y = r_bf16(__fadd_rn(bf16_to_f32(sh.xraw[res][4 * v + lane]), rf_bf16(z)));
+        if (i + 1 < L) publish(lv + kX2Off + 4 * v + lane, y, tag);
+        else a.x_out[4 * v + lane] = wt.dead ? static_cast<uint16_t>(kNanBf16) : y;
+      }
+      pp ^= 1;
+    });
   }
-  // workgroup 0 has read what every workgroup published: all have read the position and the counter
+  // workgroup 0 has read what every workgroup of the step published: all have read the position and the counter
   if (wg == 0 && tid == 0) {
+    if (ok) {
+      a.tokens[t] = tok;
+      a.docs[t] = doc_t;
+    }
     *a.t_dev = t + 1;
     a.work[0] = seq;
-    if (!dead0) __hip_atomic_store(&g_step_lock, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_load(a.work + kLockWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      __hip_atomic_store(&g_step_lock, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   }
+  return true;
+}
+
+__global__ __launch_bounds__(kThreads) void decoder_step_kernel(StepArgs a) {
+  __shared__ StepShared sh;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t old = 0;
+  if (tid == 0) old = __hip_atomic_fetch_add(a.work + kGangWord, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // the first weights, as the full gang needs them
+  StepWeights W;
+  const int i0 = step_next_att(a, 0);
+  if (i0 < a.p.layers) {
+    W.load_qkv(a.layers[i0], blockIdx.x, wave, lane);
+    W.load_proj(a.layers[i0], blockIdx.x, wave, lane);
+  }
+  W.load_fc(a.layers[0], blockIdx.x, wave, lane);
+  W.load_mp(a.layers[0], blockIdx.x, wave, lane);
+  if (tid == 0) sh.rank = old;
+  __syncthreads();
+  const uint32_t rank = __builtin_amdgcn_readfirstlane(sh.rank);
+  if (rank & kClosed) return;  // the step runs without this workgroup
+  if (step_run<true>(a, sh, W, blockIdx.x, kG)) return;
+  const int n = __builtin_amdgcn_readfirstlane(sh.gang);
+  __syncthreads();
+  step_run<false>(a, sh, W, rank & 0xffffu, n);
 }
 
 }  // namespace scope
@@ -610,7 +713,7 @@ using namespace scope;
 static int step_shape_ok(const scope_decoder_step_params* p) {
   return p && p->layers >= 2 && p->layers % 2 == 0 && p->layers / 2 <= kMaxSkip && p->H == kHeads && p->D == kHd &&
          p->dm == kDm && p->mlp == kMlp && p->bs == kBs && p->maxkv >= 1 && p->maxkv <= kMaxKv && p->T_cap >= kBs &&
-         p->T_cap % kBs == 0;
+         p->T_cap % kBs == 0 && p->workgroups >= 0 && p->workgroups <= kG;
 }
 
 extern "C" int scope_decoder_step_supported(const scope_decoder_step_params* p) {
@@ -650,9 +753,13 @@ extern "C" int scope_decoder_step(const scope_decoder_step_params* p, const scop
   StepArgs a{*p, layers, tok, t_dev, tokens, docs, embed, {ve0, ve1, ve2}, cos_t, sin_t, x_out,
              static_cast<uint32_t*>(work), host_status};
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(step_lock_kernel, dim3(1), dim3(64), 0, s, a.work, host_status, p->spin_ticks);
-  int rc = check_launch("step_lock_kernel");
+  // both launches in a row, also where streams share a hardware queue: a lock that is waited
+  // for in front of its holder's step would wait until its limit
+  static std::mutex order;
+  const std::lock_guard<std::mutex> hold(order);
+  hipLaunchKernelGGL(step_begin_kernel, dim3(1), dim3(64), 0, s, a.work);
+  int rc = check_launch("step_begin_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(decoder_step_kernel, dim3(kG), dim3(kThreads), 0, s, a);
+  hipLaunchKernelGGL(decoder_step_kernel, dim3(p->workgroups ? p->workgroups : kG), dim3(kThreads), 0, s, a);
   return check_launch("decoder_step_kernel");
 }

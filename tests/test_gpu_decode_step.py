@@ -169,3 +169,79 @@ def test_nan_reaches_the_logits(where):
     else:
         (m.k_cache if where == "key" else m.v_cache)[2][1, 60] = float("nan")
     assert bool(torch.isnan(m.step(toks[130])).all())
+
+
+@pytest.mark.parametrize("layers,window,budget", [(6, 4, 4), (16, 4, 4), (6, 20, 11)])
+def test_step_on_some_of_its_workgroups(layers, window, budget):
+    """A step that starts with some of its workgroups (no more launched, so that
+    the wait for the rest ends at its limit; with a limit of 0 the launched
+    ones that come later leave) gives the same bits as one on all 256."""
+    toks = torch.randint(0, 50256, (1152 + 24,), generator=torch.Generator().manual_seed(7)).to(DEV)
+    toks[40] = 50256
+    want = caches = None
+    for some in (False, True):
+        m = _model(1280, True, layers, window, budget, use_graph=False)
+        m.prefill(toks[:1152])
+        m.step(toks[1152:1153])
+        prm, _, work = m._fused()
+        got, seen = [], []
+        for s in range(1153, 1176):
+            launched = (0, 1, 2, 7, 71, 128, 250, 255)[s % 8] if some else 0
+            limit = 0 if some and s >= 1168 else 20_000
+            prm.workgroups, prm.gang_ticks = launched, limit
+            got.append(m.step(toks[s:s + 1]))
+            word = int(work[8:12].cpu().view(torch.int32)) & 0xFFFFFFFF
+            seen.append((word >> 16) & 0x7FFF if word >> 31 else word)
+            assert seen[-1] == (launched or 256) or (limit == 0 and 0 < seen[-1] <= (launched or 256))
+        if some:
+            print(f"  workgroups of the steps: {seen}", flush=True)
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+            assert all(x is None or torch.equal(x, y) for x, y in zip(m.k_cache + m.v_cache, caches))
+            assert int(m._t_dev) == 1176 and torch.equal(m.tokens[:1176], toks)
+        else:
+            want, caches = got, m.k_cache + m.v_cache
+
+
+_CHILD = """
+import sys, torch
+sys.path.insert(0, {root!r})
+from tests.test_gpu_decode_step import _decode_alone
+print("ready", flush=True)
+sys.stdin.readline()
+print(_decode_alone(int(sys.argv[1])), flush=True)
+"""
+
+
+def _decode_alone(seed):
+    """The tokens of three short requests (a graph after the first steps)."""
+    m = _model(512, True, 6, use_graph=True)
+    g = torch.Generator().manual_seed(seed)
+    out = []
+    for _ in range(3):
+        m.prefill(torch.randint(0, 50256, (128,), generator=g))
+        out.append(m.generate(300, 17))
+    return [t.tolist() for t in out]
+
+
+def test_two_processes_on_one_device():
+    """Two processes that decode on the same device at the same time (their
+    steps compete for the same compute units) get what one alone gets."""
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    want = _decode_alone(21)
+    print("  alone: done", flush=True)
+    child = subprocess.Popen([sys.executable, "-c", _CHILD.format(root=root), "21"], cwd=root, stdin=subprocess.PIPE,
+                             stdout=subprocess.PIPE, text=True)
+    try:
+        assert child.stdout.readline().strip() == "ready"
+        child.stdin.write("go\n")
+        child.stdin.flush()
+        print("  child started", flush=True)
+        assert _decode_alone(21) == want
+        assert child.communicate(timeout=60)[0].strip() == str(want)
+        assert child.returncode == 0
+    finally:
+        child.kill()
