@@ -354,6 +354,8 @@ __device__ __forceinline__ bool step_run(const StepArgs& a, StepShared& sh, Step
   const uint32_t seq = __hip_atomic_load(a.work, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1, tag = seq & 0xffffu;
   const bool dead0 = __hip_atomic_load(a.work + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
   StepWait wt{p.spin_ticks, a.work + 1, a.host_status, dead0};
+  if (dead0 && wg == 0 && tid == 0 && a.host_status)  // the host's copy follows the status
+    __hip_atomic_store(a.host_status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const int64_t tok = *a.tok, t = __hip_atomic_load(a.t_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const bool ok = tok >= 0 && tok < p.vocab && t >= 0 && t < p.T_cap;
   const bool pos_ok = t >= 0 && t < p.T_cap && t < p.rot_rows;

@@ -382,15 +382,21 @@ class ScopeDecoder(nn.Module):
         td.add_(1)
         return logits
 
+    def _check_waits(self, who: str) -> None:
+        """Raises if a wait inside a one-launch step that has run expired."""
+        if self._step_status is not None and int(self._step_status[0]):
+            raise RuntimeError(f"{who}: an earlier step's workgroups waited too long for each other; its logits are NaN")
+
     @torch.no_grad()
     def step(self, token: int | torch.Tensor) -> torch.Tensor:
-        """Append one token at position t; returns its logits [vocab_padded]."""
+        """Append one token at position t; returns its logits [vocab_padded]
+        (all NaN where a wait inside the one-launch step expired; the next call
+        raises then).  It does not wait for the GPU."""
         bs = self.cfg.block_size
         t = self.t
         if t >= self.max_len:
             raise ValueError("step: the cache is full")
-        if self._step_status is not None and int(self._step_status[0]):
-            raise RuntimeError("step: an earlier step's workgroups waited too long for each other; its logits are NaN")
+        self._check_waits("step")
         if not isinstance(token, torch.Tensor) or not token.is_cuda:  # a host token is checked here
             if not 0 <= int(token) < self.cfg.vocab_size:
                 raise ValueError(f"step: token {int(token)} outside the vocabulary [0, {self.cfg.vocab_size})")
@@ -430,10 +436,15 @@ class ScopeDecoder(nn.Module):
 
     @torch.no_grad()
     def generate(self, n_steps: int, first: int | torch.Tensor) -> torch.Tensor:
-        """Greedy decoding: feeds ``first``, then each argmax, for n_steps."""
+        """Greedy decoding: feeds ``first``, then each argmax, for n_steps.
+        With the one-launch step it returns when the tokens are there: a step
+        whose waits expired has no other step after it to say so."""
         out = torch.empty(n_steps, dtype=torch.int64, device=self.device)
         tok = torch.as_tensor(first, device=self.device)
         for s in range(n_steps):
             logits = self.step(tok)
             tok = ops.argmax(logits[:self.cfg.vocab_size], out=out[s:s + 1])  # written in place
+        if self._step_status is not None:
+            torch.cuda.current_stream(self.device).synchronize()
+            self._check_waits("generate")
         return out

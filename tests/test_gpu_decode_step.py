@@ -171,6 +171,22 @@ def test_nan_reaches_the_logits(where):
     assert bool(torch.isnan(m.step(toks[130])).all())
 
 
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_generate_raises_after_an_expired_wait(use_graph):
+    """The last step of a request has no step after it: generate itself says
+    that a wait expired (the status preset on the device, as such a wait
+    leaves it), instead of the token 0 that all-NaN logits give."""
+    m = _model(256, True, 6, use_graph=use_graph)
+    toks = torch.randint(0, 50256, (140,), generator=torch.Generator().manual_seed(3))
+    m.prefill(toks[:128])
+    assert bool((m.generate(6, 5) >= 0).all())
+    m._fused()[2][4:8].copy_(torch.tensor([1, 0, 0, 0], dtype=torch.uint8, device=DEV))
+    with pytest.raises(RuntimeError, match="waited too long"):
+        m.generate(1, 5)
+    m.prefill(toks[:128])
+    assert m.generate(6, 5).numel() == 6
+
+
 @pytest.mark.parametrize("layers,window,budget", [(6, 4, 4), (16, 4, 4), (6, 20, 11)])
 def test_step_on_some_of_its_workgroups(layers, window, budget):
     """A step that starts with some of its workgroups (no more launched, so that
