@@ -281,15 +281,15 @@ class ScopeDecoder(nn.Module):
                 layers.append(dict(qkv=lay.get("qkv"), proj=lay.get("proj"), mlp_fc=lay["mlp_fc"],
                                    mlp_proj=lay["mlp_proj"], k_cache=self.k_cache[i], v_cache=self.v_cache[i],
                                    kv_num=self.list_num[i], kv_idx=self.list_idx[i], ve=ve[i], va=va, vb=vb))
-            cache = next((c for c in self.k_cache if c is not None), None)
+            cache, vcache = (next((c for c in cs if c is not None), None) for cs in (self.k_cache, self.v_cache))
             self._step_table = None
-            if cache is not None and cfg.num_layers >= 6:
+            if cache is not None and vcache is not None and cfg.num_layers >= 6:
                 self._step_table = ops.decoder_step_table(layers, dict(
                     layers=cfg.num_layers, H=cfg.num_heads, D=cfg.head_dim, dm=cfg.model_dim, mlp=4 * cfg.model_dim,
                     bs=cfg.block_size, maxkv=cfg.window + cfg.budget + cfg.n_global, scale=cfg.attn_scale,
                     eps=torch.finfo(torch.float32).eps, T_cap=self.max_len, vocab=cfg.vocab_size, eot=EOT,
                     rot_rows=self.rotary.cos.shape[0], rot_st=self.rotary.cos.stride(0), k_sh=cache.stride(0),
-                    k_st=cache.stride(1), v_sh=cache.stride(0), v_st=cache.stride(1),
+                    k_st=cache.stride(1), v_sh=vcache.stride(0), v_st=vcache.stride(1),
                     spin_ticks=20 * 100_000_000, gang_ticks=50_000), cache.device)
             if self._step_status is None:
                 self._step_status = torch.zeros(1, dtype=torch.int32, pin_memory=True)

@@ -1039,8 +1039,8 @@ def decoder_step_prologue(tok: torch.Tensor, t_dev: torch.Tensor, tokens: torch.
 def decoder_step_table(layers, params: dict, device: torch.device):
     """(params struct, device table of the layer records, workspace) of
     ``decoder_step``, or None when the library's one-launch step does not
-    serve the decoder (its sizes, or a device that cannot hold the kernel's
-    workgroups at once).  ``layers``: dicts with qkv / proj (None without
+    serve the decoder (its sizes, tensors of another layout, or a device that
+    cannot hold the kernel's workgroups at once).  ``layers``: dicts with qkv / proj (None without
     attention), mlp_fc, mlp_proj, k_cache, v_cache, kv_num, kv_idx, ve, va, vb."""
     prm = _lib.DecoderStepParams(**params)
     with torch.cuda.device(device):
@@ -1048,6 +1048,10 @@ def decoder_step_table(layers, params: dict, device: torch.device):
             return None
     hd, dm, mlp = prm.H * prm.D, prm.dm, prm.mlp
     shapes = dict(qkv=(3 * hd, dm), proj=(dm, hd), mlp_fc=(mlp, dm), mlp_proj=(dm, mlp))
+    # (the strides are the step's parameters, one pair for all layers)
+    state = [("k_cache", torch.bfloat16, (prm.H, prm.T_cap, prm.D), (prm.k_sh, prm.k_st, 1)),
+             ("v_cache", torch.bfloat16, (prm.H, prm.T_cap, prm.D), (prm.v_sh, prm.v_st, 1)),
+             ("kv_num", torch.int32, (prm.H,), (1,)), ("kv_idx", torch.int32, (prm.H, prm.maxkv), (prm.maxkv, 1))]
     rec = (_lib.DecoderLayer * len(layers))()
     for r, lay in zip(rec, layers):
         for n_, shape in shapes.items():
@@ -1059,8 +1063,12 @@ def decoder_step_table(layers, params: dict, device: torch.device):
                 return None
             setattr(r, n_, w.data_ptr())
         if lay["qkv"] is not None:
-            for n_ in ("k_cache", "v_cache", "kv_num", "kv_idx"):
-                setattr(r, n_, lay[n_].data_ptr())
+            for n_, dtype, shape, stride in state:
+                t = lay[n_]
+                if t.dtype != dtype or tuple(t.shape) != shape or t.stride() != stride or t.device != device \
+                        or (dtype == torch.bfloat16 and t.data_ptr() % 16):
+                    return None
+                setattr(r, n_, t.data_ptr())
         r.ve, r.va, r.vb = lay["ve"], lay["va"], lay["vb"]
     table = torch.frombuffer(bytearray(bytes(rec)), dtype=torch.uint8).to(device)
     work = torch.zeros(int(query("scope_decoder_step_workspace_bytes", C.byref(prm))), dtype=torch.uint8, device=device)

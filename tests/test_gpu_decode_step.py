@@ -171,6 +171,35 @@ def test_nan_reaches_the_logits(where):
     assert bool(torch.isnan(m.step(toks[130])).all())
 
 
+@pytest.mark.parametrize("which", ["every v cache", "one k cache", "one list", "one list of 64 bits"])
+def test_caches_and_lists_of_another_layout(which):
+    """Caches whose rows lie otherwise in all layers are served; one that
+    differs from the others, or a list that is not contiguous int32, leaves the
+    step to the layer-by-layer kernels, with the same logits."""
+    ms = [_model(256, f, 6, use_graph=False) for f in (True, False)]
+    toks = torch.randint(0, 50256, (140,), generator=torch.Generator().manual_seed(8))
+    if which == "one list of 64 bits":
+        ms = ms[:1]
+    for m in ms:
+        if which == "every v cache":
+            m.v_cache = [c if c is None else torch.zeros_like(c.transpose(0, 1).contiguous()).transpose(0, 1)
+                         for c in m.v_cache]
+        elif which == "one k cache":
+            m.k_cache[3] = torch.zeros_like(m.k_cache[3].transpose(0, 1).contiguous()).transpose(0, 1)
+        elif which == "one list":
+            m.list_idx[3] = torch.zeros_like(m.list_idx[3].t().contiguous()).t()
+        else:
+            m.list_num[3] = m.list_num[3].long()
+        assert (m._fused() is not None) == (which == "every v cache" and m is ms[0])
+        if which.startswith("one list"):
+            return
+        m.prefill(toks[:128])
+    for s in range(128, 134):
+        a, b = (m.step(toks[s]) for m in ms)
+        assert (a - b).abs().max().item() <= (5e-2 if which == "every v cache" else 0.0)
+    _close(*ms, 134)
+
+
 @pytest.mark.parametrize("use_graph", [False, True])
 def test_generate_raises_after_an_expired_wait(use_graph):
     """The last step of a request has no step after it: generate itself says
