@@ -36,7 +36,8 @@ puts the hot-path kernels under a token loop.
 from __future__ import annotations
 
 import math
-from dataclasses import dataclass
+import operator
+from dataclasses import dataclass, replace
 
 import torch
 import torch.nn.functional as F
@@ -78,6 +79,36 @@ def _mix(a: float, b: float, x: torch.Tensor, x0: torch.Tensor) -> torch.Tensor:
 def _skip(x: torch.Tensor, w: float, s: torch.Tensor) -> torch.Tensor:
     """x + w·s (scoped_medium.py:607); w = 1 is a plain sum, exactly."""
     return x + s if w == 1.0 else x + w * s
+
+
+class _StepInputs:
+    """What a step inside a block reaches by address or bakes in, at one moment:
+    its tensors (kept alive here) and its numbers.  ``same`` compares with the
+    decoder's state now: a replaced tensor, one with other memory, and
+    (``layout``) one with other strides."""
+
+    def __init__(self, dec: "ScopeDecoder"):
+        self.tensors, self.numbers = self._of(dec)
+        self.numbers = (replace(dec.cfg), *self.numbers[1:])  # the caller's config may be changed in place
+        self.addresses = list(map(torch.Tensor.data_ptr, self.tensors))
+        self.strides = list(map(torch.Tensor.stride, self.tensors))
+
+    @staticmethod
+    def _of(dec):
+        ts = [t for lay in dec.layers for n in ("qkv", "proj", "mlp_fc", "mlp_proj") if (t := lay.get(n)) is not None]
+        for per_layer in (dec.k_cache, dec.v_cache, dec.list_num, dec.list_idx):
+            ts += [t for t in per_layer if t is not None]
+        ts += dec.value_embeds
+        ts += [dec.embed, dec.lm_head, dec.rotary.cos, dec.rotary.sin, dec.docs, dec.tokens, dec._t_dev, dec._ws]
+        return ts, (dec.cfg, list(dec.skip_weights), [(lay["lambdas"], lay.get("vlam"), "qkv" in lay)
+                                                      for lay in dec.layers])
+
+    def same(self, dec, layout: bool = True) -> bool:
+        ts, numbers = self._of(dec)
+        return (numbers == self.numbers and len(ts) == len(self.tensors)
+                and all(map(operator.is_, ts, self.tensors))
+                and list(map(torch.Tensor.data_ptr, ts)) == self.addresses
+                and (not layout or list(map(torch.Tensor.stride, ts)) == self.strides))
 
 
 class _Rotary:
@@ -147,12 +178,13 @@ class ScopeDecoder(nn.Module):
         self._ws = torch.empty(H * width * (D + 2) * 4, dtype=torch.uint8, device=device)
         self.use_graph = bool(use_graph) and self.device.type == "cuda"
         self._graph = None
+        self._g_inputs: _StepInputs | None = None  # what it was captured with
         self._g_tok = None
         self._g_out = None
         self._g_warm = 0
-        # the one-launch step (``_fused``): the table of the layers' tensors, the
-        # addresses and layouts it was made from, and the status its waits set (pinned)
-        self._step_key: tuple | None = None
+        # the one-launch step (``_fused``): the table of the layers' tensors, what
+        # it was made from, and the status its waits set (pinned)
+        self._step_inputs: _StepInputs | None = None
         self._step_table = None
         self._step_status = None
 
@@ -203,7 +235,7 @@ class ScopeDecoder(nn.Module):
             # a wait of an earlier one-launch step expired: its workspace and the
             # graph that uses it are left behind, once nothing runs on them
             torch.cuda.synchronize(self.device)
-            self._graph = self._g_table = self._step_key = self._step_table = self._step_status = None
+            self._graph = self._g_table = self._step_inputs = self._step_table = self._step_status = None
         tok = tokens.to(self.device).long()
         self.tokens[:T] = tok
         self.docs[:T] = (tok == EOT).cumsum(0).to(torch.int32)
@@ -268,12 +300,7 @@ class ScopeDecoder(nn.Module):
         if self.device.type != "cuda" or any(w != 1.0 for w in self.skip_weights) \
                 or any(lay["lambdas"] != (1.0, 0.0) for lay in self.layers) or len(self.layers) != 2 * n:
             return None
-        names = ("qkv", "proj", "mlp_fc", "mlp_proj")
-        # (an address alone could be a later tensor of another layout)
-        key = tuple((t.data_ptr(), t.dtype, t.shape, t.stride()) if t is not None else None for ts in
-                    (*([lay.get(m) for m in names] for lay in self.layers), self.k_cache, self.v_cache, self.list_num,
-                     self.list_idx) for t in ts) + tuple(lay.get("vlam", ()) for lay in self.layers)
-        if key != self._step_key:
+        if self._step_inputs is None or not self._step_inputs.same(self):
             ve = [0, 1, 2] + [-1] * (cfg.num_layers - 6) + [0, 1, 2]
             layers = []
             for i, lay in enumerate(self.layers):
@@ -293,7 +320,7 @@ class ScopeDecoder(nn.Module):
                     spin_ticks=20 * 100_000_000, gang_ticks=50_000), cache.device)
             if self._step_status is None:
                 self._step_status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-            self._step_key = key
+            self._step_inputs = _StepInputs(self)
         return self._step_table
 
     def _body(self, tok: torch.Tensor, t: int, opens: bool, closes: bool) -> torch.Tensor:
@@ -413,7 +440,11 @@ class ScopeDecoder(nn.Module):
 
     def _graph_step(self, tok: torch.Tensor, t: int) -> torch.Tensor:
         """A step inside a block: one eager run of the body first (library
-        warm-up), then a capture; every later such step replays the graph."""
+        warm-up), then a capture; every later such step replays the graph, which
+        is captured anew when what it reaches has been replaced."""
+        if self._graph is not None and not self._g_inputs.same(self, layout=False):
+            torch.cuda.synchronize(self.device)  # no replay of the old graph is running
+            self._graph = None
         if self._graph is None and self._g_warm == 0:
             self._g_warm = 1
             side = torch.cuda.Stream(self.device)
@@ -429,6 +460,7 @@ class ScopeDecoder(nn.Module):
             with torch.cuda.graph(g):
                 self._g_out = self._body(self._g_tok, -1, False, False)
             self._graph = g  # the capture ran nothing: replay for this token below
+            self._g_inputs = _StepInputs(self)
         else:
             self._g_tok.copy_(tok)
         self._graph.replay()

@@ -200,6 +200,45 @@ def test_caches_and_lists_of_another_layout(which):
     _close(*ms, 134)
 
 
+@pytest.mark.parametrize("what,fused", [("weight", True), ("cache", True), ("lists", True), ("scale", True),
+                                        ("lambdas", True), ("data", True), ("weight", False), ("vlam", False),
+                                        ("lm_head", False)])
+def test_replays_see_what_was_replaced(what, fused):
+    """After a capture, a step inside a block uses the decoder's tensors and
+    numbers of that moment, as an eager step does."""
+    ms = [_model(256, fused, 6, use_graph=g) for g in (True, False)]
+    toks = torch.randint(0, 50256, (150,), generator=torch.Generator().manual_seed(10))
+    for m in ms:
+        m.prefill(toks[:128])
+    for s in range(128, 134):
+        a, b = (m.step(toks[s]) for m in ms)
+    assert ms[0]._graph is not None and torch.equal(a, b)
+    old = []
+    for m in ms:
+        lay = m.layers[2]
+        old.append((lay["mlp_fc"], m.k_cache[1], m.list_idx[1], m.lm_head))
+        if what == "weight":
+            lay["mlp_fc"] = -lay["mlp_fc"]
+        elif what == "data":
+            lay["mlp_fc"].data = -lay["mlp_fc"]
+        elif what == "cache":
+            m.k_cache[1] = -m.k_cache[1]
+        elif what == "lists":
+            m.list_num[1] = torch.zeros_like(m.list_num[1])
+        elif what == "scale":
+            m.cfg.attn_scale = 0.5
+        elif what == "vlam":
+            lay["vlam"] = (0.25, -0.5)
+        elif what == "lambdas":
+            lay["lambdas"] = (0.5, 1.0)
+        else:
+            m.lm_head = -m.lm_head
+    for s in range(134, 139):
+        a, b = (m.step(toks[s]) for m in ms)
+        assert torch.equal(a, b), f"position {s}"
+    _close(*ms, 139)
+
+
 @pytest.mark.parametrize("use_graph", [False, True])
 def test_generate_raises_after_an_expired_wait(use_graph):
     """The last step of a request has no step after it: generate itself says
