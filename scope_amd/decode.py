@@ -301,6 +301,8 @@ class ScopeDecoder(nn.Module):
                 or any(lay["lambdas"] != (1.0, 0.0) for lay in self.layers) or len(self.layers) != 2 * n:
             return None
         if self._step_inputs is None or not self._step_inputs.same(self):
+            if self._step_table is not None:  # left behind once no step runs on it, on whatever stream
+                torch.cuda.synchronize(self.device)
             ve = [0, 1, 2] + [-1] * (cfg.num_layers - 6) + [0, 1, 2]
             layers = []
             for i, lay in enumerate(self.layers):
@@ -447,6 +449,7 @@ class ScopeDecoder(nn.Module):
             self._graph = None
         if self._graph is None and self._g_warm == 0:
             self._g_warm = 1
+            self._fused()  # its table and workspace belong to the caller's stream, not to the side stream
             side = torch.cuda.Stream(self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
             with torch.cuda.stream(side):

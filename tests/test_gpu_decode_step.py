@@ -239,6 +239,27 @@ def test_replays_see_what_was_replaced(what, fused):
     _close(*ms, 139)
 
 
+def test_table_and_workspace_belong_to_the_callers_stream():
+    """They are used on the caller's stream from then on: allocated on the
+    warm-up's side stream, their memory could go to new tensors of that stream
+    while a step still used it."""
+    m = _model(256, True, 6, use_graph=True)
+    toks = torch.randint(0, 50256, (140,), generator=torch.Generator().manual_seed(11))
+    m.prefill(toks[:128])
+    caller = torch.cuda.Stream()
+    caller.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(caller):
+        for s in range(128, 133):
+            m.step(toks[s])
+    torch.cuda.synchronize()
+    streams = {}
+    for seg in torch.cuda.memory_snapshot():
+        for t in m._step_table[1:]:
+            if seg["address"] <= t.data_ptr() < seg["address"] + seg["total_size"]:
+                streams[t.data_ptr()] = seg["stream"]
+    assert list(streams.values()) == [caller.cuda_stream] * 2
+
+
 @pytest.mark.parametrize("use_graph", [False, True])
 def test_generate_raises_after_an_expired_wait(use_graph):
     """The last step of a request has no step after it: generate itself says
