@@ -37,6 +37,7 @@ from __future__ import annotations
 
 import math
 import operator
+import threading
 from dataclasses import dataclass, replace
 
 import torch
@@ -46,6 +47,12 @@ from torch import nn
 from . import ops
 
 EOT = 50256
+
+# Held while a step's launches are enqueued (a graph's as well as single ones):
+# the launch that takes the step lock and the step behind it come in a row also
+# where the streams of two threads share a hardware queue.  A lock waited for in
+# front of its holder's step would be waited for until its limit.
+_ENQUEUE = threading.Lock()
 
 
 @dataclass
@@ -334,8 +341,9 @@ class ScopeDecoder(nn.Module):
         td = self._t_dev
         fused = None if opens else self._fused()
         if fused is not None:
-            x = ops.decoder_step(*fused, tok, td, self.tokens, self.docs, self.embed, self.value_embeds,
-                                 self.rotary.cos, self.rotary.sin, self._step_status)
+            with _ENQUEUE:
+                x = ops.decoder_step(*fused, tok, td, self.tokens, self.docs, self.embed, self.value_embeds,
+                                     self.rotary.cos, self.rotary.sin, self._step_status)
             if closes:  # the block is complete: its key means join the candidates
                 for kbar, kc in zip(self.kbar, self.k_cache):
                     if kbar is not None:
@@ -466,7 +474,8 @@ class ScopeDecoder(nn.Module):
             self._g_inputs = _StepInputs(self)
         else:
             self._g_tok.copy_(tok)
-        self._graph.replay()
+        with _ENQUEUE:
+            self._graph.replay()
         return self._g_out.clone()
 
     @torch.no_grad()

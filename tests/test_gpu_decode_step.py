@@ -307,6 +307,37 @@ def test_step_on_some_of_its_workgroups(layers, window, budget):
             want, caches = got, m.k_cache + m.v_cache
 
 
+def test_two_threads_replaying_on_streams_of_their_own():
+    """Two decoders driven by two threads (each replay takes the step lock and
+    runs the step) give what each gives alone."""
+    import threading
+
+    g = torch.Generator().manual_seed(12)
+    toks = [torch.randint(0, 50256, (128 + 120,), generator=g).to(DEV) for _ in range(2)]
+    ms = [_model(256, True, 6, use_graph=True) for _ in range(2)]
+
+    def request(i):
+        ms[i].prefill(toks[i][:128])
+        return torch.stack([ms[i].step(t) for t in toks[i][128:].split(1)])
+
+    want = [request(i) for i in range(2)]  # the graphs are captured here
+    torch.cuda.synchronize()
+    got, streams = [None, None], [torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def work(i):
+        with torch.cuda.stream(streams[i]), torch.no_grad():
+            for _ in range(3):
+                got[i] = request(i)
+            streams[i].synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 _CHILD = """
 import sys, torch
 sys.path.insert(0, {root!r})
