@@ -138,7 +138,7 @@ __device__ __forceinline__ void coeff_sincos(float x, bool slow, float& s, float
   else sincos_reduced(x, s, c);
 }
 
-// e^-x of a finite x >= 0 as 2^(-x log2 e): log2 e as the sum of two floats, the
+// e^-x of x in [0, 1e9] as 2^(-x log2 e): log2 e as the sum of two floats, the
 // first product's rounding error carried by an fma, the integer part to the exponent
 __device__ __forceinline__ float exp_neg(float x) {
   const float t = x * -1.44269502f;  // -log2 e, and its remainder below
@@ -148,9 +148,15 @@ __device__ __forceinline__ float exp_neg(float x) {
 }
 
 // e_mk for one peak (the caller normalises); den = 2 s_m², rden = 1 / den: the
-// quotient with one correction step is the division's but for rare last bits
+// quotient with one correction step is the division's but for rare last bits.
+// An infinite log ω_k (a band at ω = 0; fp32 frequencies end at -104 and 89) is
+// taken as ±1e4: e_mk = 0 as from the infinity itself, but the square stays where
+// exp_neg's integer part is one.  On the bits, which the scalar unit compares
+// (log ω_k is the same in every lane; as floats: 1% of the head).
 __device__ __forceinline__ float coeff_e(const float* logw, int k, float mu, float den, float rden) {
-  const float d = logw[k] - mu, dd = d * d;
+  const uint32_t lw = __float_as_uint(logw[k]);
+  const uint32_t lf = (lw & 0x7fffffffu) == 0x7f800000u ? (lw & 0x80000000u) | 0x461c4000u : lw;
+  const float d = __uint_as_float(lf) - mu, dd = d * d;
   const float q = dd * rden;
   return exp_neg(fmaf(fmaf(-q, den, dd), rden, q));
 }

@@ -202,3 +202,28 @@ def test_disabled_forward_on_gpu():
     assert len(out) == 12 and out[0].is_cuda
     assert all(torch.all(out[i] == 0) for i in (0, 1, 2, 3, 4, 6, 7, 8, 11))
     assert torch.allclose(out[5], torch.full_like(out[5], 1 / 3))
+
+
+@pytest.mark.parametrize("where", [0, 3])
+def test_band_at_frequency_zero(where):
+    """A band at ω = 0 has log ω = -inf: its weight e_mk is 0 in every peak,
+    its coefficients are 0 and the others those of the head without it (five
+    and six bands are two instantiations of the kernel, whose sums may be
+    contracted differently: up to eight roundings of values of at most 1 in a
+    coefficient, 2^-21, and five more in b0)."""
+    from scope_amd import ops
+
+    g = torch.Generator().manual_seed(3)
+    M, K, L, H = 8, 6, 256, 2
+    y = (torch.randn((1, H, L, 5 * M + 1), generator=g) * 2).to(DEV)
+    om = torch.logspace(-4.5, -1.0, K).to(DEV)
+    om[where] = 0.0
+    keep = [k for k in range(K) if k != where]
+    a = ops.coeff_head_fwd(y, _prm(M, K, L, False), om, om.log(), None, None)
+    b = ops.coeff_head_fwd(y, _prm(M, K - 1, L, False), om[keep].contiguous(), om[keep].log(), None, None)
+    for n in ("coeff_cos", "coeff_sin"):
+        assert bool((a[n][..., where] == 0).all()), n
+        assert (a[n][..., keep] - b[n]).abs().max().item() <= 2.0 ** -21, n
+    assert (a["b0"] - b["b0"]).abs().max().item() <= 2.0 ** -20
+    for n in ("slope", "pi", "width", "delta_main"):
+        assert torch.equal(a[n], b[n]), n
