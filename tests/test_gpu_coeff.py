@@ -227,3 +227,42 @@ def test_band_at_frequency_zero(where):
     assert (a["b0"] - b["b0"]).abs().max().item() <= 2.0 ** -20
     for n in ("slope", "pi", "width", "delta_main"):
         assert torch.equal(a[n], b[n]), n
+
+
+@pytest.mark.parametrize("top", [60000.0, 65535.0, 65537.0, 1.0e6, 3.0e7])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_sine_and_cosine_at_large_phases(top, mixed):
+    """Phases up to ``top`` on both sides of the limit of the two-step
+    reduction (65536), with rows of small phases in the same wavefront
+    (``mixed``): one peak (π = 1) and one band (a = 1), so that coeff_cos and
+    coeff_sin are the sine and cosine of the row's fp32 phase ω·Δ*.
+
+    The head returns Δ*, so the phase is known to the bit; the bar is the error
+    written at the functions, 7.2e-8, plus the roundings after it: the product
+    with π·a (2^-24); in the gradient eight products (2^-24 each, relative) and
+    the fp32 1 - σ, where σ is 2^-23 off."""
+    from scope_amd import ops
+
+    g = torch.Generator().manual_seed(int(top))
+    M, K, L, H = 1, 1, 4096, 2
+    y = (torch.randn((1, H, L, 5 * M + 1), generator=g) * 3).to(DEV)
+    y[..., 1:] = 0.0  # μ, σ and the rest at their middle
+    if mixed:
+        y[:, :, ::3, 0] = -14.0  # σ about 1e-6
+    prm = _prm(M, K, L, False)
+    prm.update(delta_cap=float(L - 1), use_slope=False)
+    om = torch.tensor([top / (L - 1)], dtype=torch.float32, device=DEV)
+    out = ops.coeff_head_fwd(y, prm, om, torch.full((1,), -7.0, device=DEV), None, None)
+    ds = out["delta_star"][..., 0]
+    ph = (om * ds).double()  # the product rounded to fp32, as in the head
+    assert ph.max().item() > 0.9 * top and (not mixed or ph.min().item() < 1e-3 * top)
+    for n, ref in (("coeff_cos", ph.cos()), ("coeff_sin", ph.sin())):
+        err = (out[n][..., 0].double() - ref).abs().max().item()
+        assert err <= 7.2e-8 + 2.0 ** -24, f"{n}: {err:.3e}"
+    # d coeff_cos / d delta_raw = -sin(phase)·ω·Δ*·(1 - σ) (and cos for coeff_sin), from the backward's own pair
+    for n, f in (("coeff_cos", lambda x: -x.sin()), ("coeff_sin", lambda x: x.cos())):
+        dy = ops.coeff_head_bwd(y, prm, om, torch.full((1,), -7.0, device=DEV), None, None,
+                                {n: torch.ones_like(out[n])}, None, out["reg"])
+        rest = 1 - torch.sigmoid(y[..., 0].double())
+        err = (dy[..., 0].double() - f(ph) * ph * rest).abs() / (ph * rest)
+        assert bool((err <= 7.2e-8 + 8 * 2.0 ** -24 + 2.0 ** -22 / rest).all()), f"d{n}: {err.max().item():.3e}"
