@@ -141,6 +141,7 @@ __device__ __forceinline__ void coeff_sincos(float x, bool slow, float& s, float
 // e^-x of x in [0, 1e9] as 2^(-x log2 e): log2 e as the sum of two floats, the
 // first product's rounding error carried by an fma, the integer part to the exponent
 __device__ __forceinline__ float exp_neg(float x) {
+#pragma clang fp contract(off)  // t - n as a fused multiply-add of x would count t's rounding error, which lo holds, twice
   const float t = x * -1.44269502f;  // -log2 e, and its remainder below
   const float lo = fmaf(x, -1.92596303e-8f, fmaf(x, -1.44269502f, -t));
   const float n = rintf(t);
