@@ -675,11 +675,11 @@ __device__ __forceinline__ void dkv16_probs(const AttnArgs& a, const DkvBuf<MODE
       float x;
       if constexpr (TOK) {
         const float df = dfb + static_cast<float>(i);  // q - wkv, exact in fp32
-        float e = fmaf(slv[i], df, ofv[i]);
+        float e = GATE ? slv[i] * df : fmaf(slv[i], df, ofv[i]);
         if constexpr (GATE) {
           const float y = gate_y(df - dmv[i], wdv[i], a.inv_tau * kLog2e);
           const float spw = a.gate_kind == SCOPE_GATE_SOFTPLUS ? 1.f : 0.f;
-          e = fmaf(-a.beta_log2 * a.ramp_lambda * kLn2, gate_g(y, 1.f + gate_en(y, spw)), e);
+          e = fmaf(-a.beta_log2 * a.ramp_lambda * kLn2, gate_g(y, 1.f + gate_en(y, spw)), e) + ofv[i];
         }
         x = fmaf(s[mb][i], cs, e);
       } else {
@@ -1274,7 +1274,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             float sig = 0.f, ssig = 0.f, df = 0.f;  // the gate's slope in |Δ - δ|, and in Δ - δ
             if (TOK) {
               df = dfl - static_cast<float>(16 * kb4 + r);  // lim - j, exact in fp32
-              float e = fmaf(slp, df, off);
+              float e = GATE ? slp * df : fmaf(slp, df, off);
               if (GATE) {
                 const float dd = df - dm;
                 const float y = gate_y(dd, wd, y_scale);
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 const float inv = __builtin_amdgcn_rcpf(en1);
                 sig = y > 0.f ? inv : en * inv;
                 ssig = dd != 0.f ? copysignf(sig, dd) : 0.f;
-                e = fmaf(-glam, gate_g(y, en1), e);
+                e = fmaf(-glam, gate_g(y, en1), e) + off;  // the large offset last: it rounds coarsest
               }
               x = fmaf(s[kl][r], cs, e);
             } else {

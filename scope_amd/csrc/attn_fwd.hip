@@ -78,10 +78,13 @@ __device__ __forceinline__ void fwd_scores(const AttnArgs& a, const Tile& b, con
         float x;
         if (TOK) {
           const float jc = static_cast<float>(mb * 32 + 8 * rq + i);
-          float e = fmaf(-R.slp, jc, sbase);
+          float e;
           if (GATE) {
-            const float y = gate_y((dfl - jc) - R.dm, R.wd, y_scale);
-            e = fmaf(-glam, gate_g(y, 1.f + gate_en(y, spw)), e);
+            const float df = dfl - jc;  // exact
+            const float y = gate_y(df - R.dm, R.wd, y_scale);
+            e = fmaf(-glam, gate_g(y, 1.f + gate_en(y, spw)), R.slp * df);
+          } else {
+            e = fmaf(-R.slp, jc, sbase);
           }
           x = fmaf(s[mb][r], cs, e);
         } else {
