@@ -24,11 +24,24 @@ def _model(max_len, fused=True, layers=16, window=4, budget=4, **kw):
 
 
 def _close(a, b, t):
-    err = max((x[:, :t].float() - y[:, :t].float()).abs().max().item() for x, y in zip(a.k_cache + a.v_cache,
-              b.k_cache + b.v_cache) if x is not None)
-    assert err <= 2.0 ** -4, f"cache difference {err:.3e}"
-    err = max((x - y).abs().max().item() for x, y in zip(a.kbar, b.kbar) if x is not None)
-    assert err <= 2.0 ** -4, f"key-mean difference {err:.3e}"
+    for i, (x, y) in enumerate(zip(a.k_cache + a.v_cache, b.k_cache + b.v_cache)):
+        if x is not None:  # (a NaN fails every comparison here)
+            err = (x[:, :t].float() - y[:, :t].float()).abs().max().item()
+            assert err <= 2.0 ** -4, f"cache {i}: difference {err:.3e}"
+    for i, (x, y) in enumerate(zip(a.kbar, b.kbar)):
+        if x is not None:
+            err = (x - y).abs().max().item()
+            assert err <= 2.0 ** -4, f"key means {i}: difference {err:.3e}"
+
+
+def _logits_close(a, b, what):
+    """Elementwise 5e-2, and 3e-2 of the spread about the logits' middle (15) in
+    the 2-norm: bf16 values that round to a neighbour at sixteen layers' places
+    show up to 1e-2 there.  Returns the largest difference."""
+    assert bool(torch.isfinite(a).all()) and bool(torch.isfinite(b).all()), what
+    d, rel = (a - b).abs().max().item(), ((a - b).norm() / (b - 15).norm()).item()
+    assert d <= 5e-2 and rel <= 3e-2, f"{what}: {d:.3e}, {rel:.3e} of the spread"
+    return d, rel
 
 
 @pytest.mark.parametrize("layers,window,budget,T0,n", [(16, 4, 4, 256, 133), (8, 2, 1, 128, 9), (6, 20, 11, 1152, 5)])
@@ -43,15 +56,13 @@ def test_step_equals_layer_by_layer(layers, window, budget, T0, n):
     assert one._fused() is not None
     for m in (one, ref):
         m.prefill(toks[:T0])
-    worst = 0.0
+    worst = (0.0, 0.0)
     for s in range(n):
-        a, b = one.step(toks[T0 + s]), ref.step(toks[T0 + s])
-        worst = max(worst, (a - b).abs().max().item())
-        assert worst <= 5e-2, f"step {s}: {worst:.3e}"
+        worst = max(worst, _logits_close(one.step(toks[T0 + s]), ref.step(toks[T0 + s]), f"step {s}"))
     assert torch.equal(one.docs, ref.docs) and torch.equal(one.tokens, ref.tokens)
     assert int(one._t_dev) == int(ref._t_dev) == T0 + n
     _close(one, ref, T0 + n)
-    print(f"  max logit difference {worst:.3e}", flush=True)
+    print(f"  max logit difference {worst[0]:.3e}, there {worst[1]:.3e} of the spread", flush=True)
 
 
 def test_token_outside_the_vocabulary_and_other_sizes():
@@ -64,8 +75,7 @@ def test_token_outside_the_vocabulary_and_other_sizes():
     for m in (one, ref):
         m.prefill(toks[:128])
         m.step(toks[128])
-    a, b = one.step(bad), ref.step(bad)
-    assert (a - b).abs().max().item() <= 5e-2
+    _logits_close(one.step(bad), ref.step(bad), "bad token")
     assert torch.equal(one.docs, ref.docs) and torch.equal(one.tokens, ref.tokens)
     from scope_amd.decode import DecoderConfig, ScopeDecoder
 
@@ -146,8 +156,7 @@ def test_token_outside_the_vocabulary_stays_in_its_document():
         m.step(toks[128])
     for s in range(129, 135):
         tok = bad if s == 131 else toks[s]
-        a, b = one.step(tok), ref.step(tok)
-        assert (a - b).abs().max().item() <= 5e-2, f"position {s}"
+        _logits_close(one.step(tok), ref.step(tok), f"position {s}")
     assert torch.equal(one.docs, ref.docs)
     _close(one, ref, 135)
 
@@ -196,7 +205,8 @@ def test_caches_and_lists_of_another_layout(which):
         m.prefill(toks[:128])
     for s in range(128, 134):
         a, b = (m.step(toks[s]) for m in ms)
-        assert (a - b).abs().max().item() <= (5e-2 if which == "every v cache" else 0.0)
+        _logits_close(a, b, f"position {s}")
+        assert which == "every v cache" or torch.equal(a, b)
     _close(*ms, 134)
 
 
