@@ -28,8 +28,10 @@ import json
 import os
 import sys
 
-KERNELS = ("attn_fwd_kernel", "attn_fwd_kernel(lse)", "attn_fwd_kernel(mass)", "attn_bwd_dq2_kernel",
-           "attn_bwd_dq16_kernel", "attn_bwd_dq_kernel", "attn_bwd_dkv16_kernel", "bwd_reduce_kernel", "block_means_kernel", "ptr_logits_kernel", "ptr_score_kernel",
+KERNELS = ("attn_fwd_kernel", "attn_fwd_kernel(lse)", "attn_fwd_kernel(mass)", "attn_fwd_kernel(entry sums)",
+           "mass_merge_kernel", "attn_bwd_dq2_kernel", "attn_bwd_dq16_kernel", "attn_bwd_dq_kernel",
+           "attn_bwd_dkv16_kernel", "bwd_reduce_kernel", "block_means_kernel", "ptr_logits_kernel", "ptr_score_kernel",
+           "decoder_step_kernel", "step_begin_kernel",
            "stats_kernel", "tr_fill_kernel", "tr_sort_kernel", "tr_count_kernel", "swa_count_kernel",
            "swa_rows_kernel", "swa_pad_kernel", "coeff_fwd_kernel", "coeff_bwd_kernel", "coeff_reg_kernel",
            "probe_mfma_kernel", "probe_copy_kernel")
