@@ -128,7 +128,9 @@ def teacher_block_mass(q: torch.Tensor, k: torch.Tensor, docs: torch.Tensor, *, 
     block's keys -> [H, NB, NB] fp32.  The reference builds the same scores
     from bf16 q / k and augmented q_pos / k_pos features (the band term and
     slope of ``spectral``, offset="token"); here the bias is evaluated as in
-    ``scope_attention``.  q, k: [1,H,T,D] bf16 (the teacher's selected heads)."""
+    ``scope_attention``.  q, k: [1,H,T,D] bf16 (the teacher's selected heads).
+    The call takes a workspace of 8 bytes per row and listed block, at most
+    256 MiB, from torch's allocator."""
     from .blockmask import ScopeBlockMask  # noqa: F401  (same mask conventions)
 
     T = q.shape[-2]

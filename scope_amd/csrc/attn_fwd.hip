@@ -144,7 +144,6 @@ __global__ __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int per = (a.part_rows + 7) / 8, x = blockIdx.x % 8, j = blockIdx.x / 8;
     row = (j % per) * 8 + x;
     if (row >= a.part_rows) return;
-    e0 = j / per * a.part_entries;
     row += a.part_row0;
     e0 = j / per * a.part_entries;
   } else {
@@ -752,11 +751,12 @@ extern "C" int64_t scope_attn_block_mass_workspace_bytes(const scope_attn_params
 // workgroup each, that write every row's (maximum, sum) per entry; a second
 // kernel forms the LSE and the masses of a row from them.  Against the
 // two-pass kernels (LSE, then masses) it forms the scores once, and a
-// q-block's list is no longer one workgroup's serial chain: at T = 16384, H = 4
-// the two passes took 291 + 330 us (their 512 workgroups are all resident from
-// the start, so the longest list is the time), this takes 220 + 22; the
-// teacher's call 629 -> 250 us there, 664 -> 118 at H = 1, 2456 -> 1560 at
-// T = 65536, H = 8.  What bounds it now is the scores' VALU work (about 170
+// q-block's list is no longer one workgroup's serial chain (at T = 16384, H = 4
+// the two passes' 512 workgroups are all resident from the start, so the longest
+// list was the time).  teacher_block_mass with one document, K = 6 and a slope:
+// T = 16384, H = 4 737 -> 303 us, H = 1 654 -> 109; T = 65536, H = 8
+// 15.15 -> 7.93 ms; with two documents, T = 16384, H = 4 593 -> 201 us.  What
+// bounds it now is the scores' VALU work (about 170
 // instructions and 32 exponentials per 64-key tile and wavefront for 22 MFMAs).
 extern "C" int scope_attn_block_mass_ws(const scope_attn_params* p, const uint16_t* q, const uint16_t* k,
                                         const int32_t* kv_num, const int32_t* kv_idx, const int32_t* docs,
