@@ -326,7 +326,7 @@ class ScopeDecoder(nn.Module):
                     eps=torch.finfo(torch.float32).eps, T_cap=self.max_len, vocab=cfg.vocab_size, eot=EOT,
                     rot_rows=self.rotary.cos.shape[0], rot_st=self.rotary.cos.stride(0), k_sh=cache.stride(0),
                     k_st=cache.stride(1), v_sh=vcache.stride(0), v_st=vcache.stride(1),
-                    spin_ticks=20 * 100_000_000, gang_ticks=50_000), cache.device)
+                    spin_ticks=20 * 100_000_000, gang_ticks=50_000), cache.device)  # 20 s; 0.5 ms, about a step
             if self._step_status is None:
                 self._step_status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
             self._step_inputs = _StepInputs(self)
