@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define SCOPE_ABI_VERSION 3
+#define SCOPE_ABI_VERSION 4
 
 enum {
   SCOPE_OK = 0,
