@@ -1049,6 +1049,7 @@ def decoder_step_table(layers, params: dict, device: torch.device):
     hd, dm, mlp = prm.H * prm.D, prm.dm, prm.mlp
     shapes = dict(qkv=(3 * hd, dm), proj=(dm, hd), mlp_fc=(mlp, dm), mlp_proj=(dm, mlp))
     # (the strides are the step's parameters, one pair for all layers)
+    # a cache may be longer than the T_cap rows the step uses
     state = [("k_cache", torch.bfloat16, (prm.H, prm.T_cap, prm.D), (prm.k_sh, prm.k_st, 1)),
              ("v_cache", torch.bfloat16, (prm.H, prm.T_cap, prm.D), (prm.v_sh, prm.v_st, 1)),
              ("kv_num", torch.int32, (prm.H,), (1,)), ("kv_idx", torch.int32, (prm.H, prm.maxkv), (prm.maxkv, 1))]
@@ -1065,6 +1066,8 @@ def decoder_step_table(layers, params: dict, device: torch.device):
         if lay["qkv"] is not None:
             for n_, dtype, shape, stride in state:
                 t = lay[n_]
+                if dtype == torch.bfloat16:
+                    t = t[:, :prm.T_cap]
                 if t.dtype != dtype or tuple(t.shape) != shape or t.stride() != stride or t.device != device \
                         or (dtype == torch.bfloat16 and t.data_ptr() % 16):
                     return None
