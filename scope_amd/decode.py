@@ -38,7 +38,7 @@ from __future__ import annotations
 import math
 import operator
 import threading
-from dataclasses import dataclass, replace
+from dataclasses import dataclass
 
 import torch
 import torch.nn.functional as F
@@ -88,6 +88,10 @@ def _skip(x: torch.Tensor, w: float, s: torch.Tensor) -> torch.Tensor:
     return x + s if w == 1.0 else x + w * s
 
 
+_CFG_NUMBERS = operator.attrgetter("attn_scale", "block_size", "num_layers", "num_heads", "head_dim", "model_dim",
+                                   "vocab_size", "window", "budget", "n_global")
+
+
 class _StepInputs:
     """What a step inside a block reaches by address or bakes in, at one moment:
     its tensors (kept alive here) and its numbers.  ``same`` compares with the
@@ -96,7 +100,6 @@ class _StepInputs:
 
     def __init__(self, dec: "ScopeDecoder"):
         self.tensors, self.numbers = self._of(dec)
-        self.numbers = (replace(dec.cfg), *self.numbers[1:])  # the caller's config may be changed in place
         self.addresses = list(map(torch.Tensor.data_ptr, self.tensors))
         self.strides = list(map(torch.Tensor.stride, self.tensors))
 
@@ -107,8 +110,8 @@ class _StepInputs:
             ts += [t for t in per_layer if t is not None]
         ts += dec.value_embeds
         ts += [dec.embed, dec.lm_head, dec.rotary.cos, dec.rotary.sin, dec.docs, dec.tokens, dec._t_dev, dec._ws]
-        return ts, (dec.cfg, list(dec.skip_weights), [(lay["lambdas"], lay.get("vlam"), "qkv" in lay)
-                                                      for lay in dec.layers])
+        return ts, (_CFG_NUMBERS(dec.cfg), tuple(dec.skip_weights),
+                    [(tuple(lay["lambdas"]), tuple(lay.get("vlam", ())), "qkv" in lay) for lay in dec.layers])
 
     def same(self, dec, layout: bool = True) -> bool:
         ts, numbers = self._of(dec)

@@ -180,9 +180,9 @@ def test_nan_reaches_the_logits(where):
     assert bool(torch.isnan(m.step(toks[130])).all())
 
 
-@pytest.mark.parametrize("which", ["every v cache", "one k cache", "one list", "one list of 64 bits"])
+@pytest.mark.parametrize("which", ["every v cache", "one k cache", "longer caches", "one list", "one list of 64 bits"])
 def test_caches_and_lists_of_another_layout(which):
-    """Caches whose rows lie otherwise in all layers are served; one that
+    """Caches whose rows lie otherwise, or are more, in all layers are served; one that
     differs from the others, or a list that is not contiguous int32, leaves the
     step to the layer-by-layer kernels, with the same logits."""
     ms = [_model(256, f, 6, use_graph=False) for f in (True, False)]
@@ -193,25 +193,29 @@ def test_caches_and_lists_of_another_layout(which):
         if which == "every v cache":
             m.v_cache = [c if c is None else torch.zeros_like(c.transpose(0, 1).contiguous()).transpose(0, 1)
                          for c in m.v_cache]
+        elif which == "longer caches":
+            m.k_cache, m.v_cache = ([c if c is None else torch.zeros((8, 512, 128), dtype=c.dtype, device=DEV)
+                                     for c in cs] for cs in (m.k_cache, m.v_cache))
         elif which == "one k cache":
             m.k_cache[3] = torch.zeros_like(m.k_cache[3].transpose(0, 1).contiguous()).transpose(0, 1)
         elif which == "one list":
             m.list_idx[3] = torch.zeros_like(m.list_idx[3].t().contiguous()).t()
         else:
             m.list_num[3] = m.list_num[3].long()
-        assert (m._fused() is not None) == (which == "every v cache" and m is ms[0])
+        served = which in ("every v cache", "longer caches")
+        assert (m._fused() is not None) == (served and m is ms[0])
         if which.startswith("one list"):
             return
         m.prefill(toks[:128])
     for s in range(128, 134):
         a, b = (m.step(toks[s]) for m in ms)
         _logits_close(a, b, f"position {s}")
-        assert which == "every v cache" or torch.equal(a, b)
+        assert served or torch.equal(a, b)
     _close(*ms, 134)
 
 
 @pytest.mark.parametrize("what,fused", [("weight", True), ("cache", True), ("lists", True), ("scale", True),
-                                        ("lambdas", True), ("data", True), ("weight", False), ("vlam", False),
+                                        ("lambdas", True), ("vlam in place", True), ("data", True), ("weight", False), ("vlam", False),
                                         ("lm_head", False)])
 def test_replays_see_what_was_replaced(what, fused):
     """After a capture, a step inside a block uses the decoder's tensors and
@@ -219,6 +223,7 @@ def test_replays_see_what_was_replaced(what, fused):
     ms = [_model(256, fused, 6, use_graph=g) for g in (True, False)]
     toks = torch.randint(0, 50256, (150,), generator=torch.Generator().manual_seed(10))
     for m in ms:
+        m.layers[2]["vlam"] = [0.5, 0.5]
         m.prefill(toks[:128])
     for s in range(128, 134):
         a, b = (m.step(toks[s]) for m in ms)
@@ -239,6 +244,8 @@ def test_replays_see_what_was_replaced(what, fused):
             m.cfg.attn_scale = 0.5
         elif what == "vlam":
             lay["vlam"] = (0.25, -0.5)
+        elif what == "vlam in place":
+            lay["vlam"][0] = 0.25
         elif what == "lambdas":
             lay["lambdas"] = (0.5, 1.0)
         else:
