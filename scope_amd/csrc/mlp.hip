@@ -303,7 +303,7 @@ __device__ __forceinline__ const uint16_t* mlp_wave_rows(const MlpArgs& g, int64
 // 32 rows for 2 bytes each (24 stores a lane forward, 32 loads backward).  At a
 // million rows the forward went from 184 to 174 us and the row-wise backward
 // from 354 to 332, the weight-gradient kernel beside them unchanged (336, 359:
-// the second figure on a slower box).
+// the second figure on a slower machine).
 
 // Outputs 16ks + 8gq .. +7 of a row as bf16 pairs; past O whatever follows
 // (up to 15 outputs), which mlp_gy_mask clears: apart, so that nothing waits
@@ -366,7 +366,7 @@ __device__ __forceinline__ void bf16_round2(float& a, float& b) {
 // rounded one by one and the derivative as σ·(1 + z·(1 - σ))).  With it, the
 // 32-bit row split and db2 shared among the hidden blocks, the head at a
 // million rows, forward and backward, went from 1/1.063 to 1/1.108 of a fixed
-// older build timed beside it (1214 us on a slow box).
+// older build timed beside it (1214 us on a slow machine).
 __device__ __forceinline__ void mlp_silu_bwd2(float z0, float z1, float dx0, float dx1, float (&xv)[2],
                                               float (&dv)[2]) {
   bf16_round2(z0, z1);

@@ -65,7 +65,7 @@ class _Operator:
     up one by one, and there are none here).  A training layer's dozen
     operators were bound by that below T = 8192 or so: a step of the
     reference's default layer at T = 2176, H = 8 took 1.28 times as long
-    (976 and 765 us in turn on one box)."""
+    (976 and 765 us in turn on one machine)."""
 
     def __init__(self, name, fn):
         self._name = name
