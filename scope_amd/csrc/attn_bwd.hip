@@ -619,7 +619,7 @@ __device__ __forceinline__ int drop_masked_rows(const AttnArgs& a, int ne, int h
 // instructions a score, four of them transcendental); its gate terms are
 // scheduled one row block at a time, or the registers of two wavefronts per
 // SIMD would not hold them.  At T=16384, H=8, lists of 14, one document it
-// takes 386 us; 32 keys per wavefront, one wavefront per SIMD, took 506.  Per 64-row query tile a wavefront computes, with
+// takes 390 us; 32 keys per wavefront, one wavefront per SIMD, took 506.  Per 64-row query tile a wavefront computes, with
 // v_mfma_f32_16x16x32_bf16:
 //   S = Q·K^T, dP = dO·V^T   (M = 16 query rows × 4, N = its 16 keys, K and V
 //                             of those keys held in registers as B operands)

@@ -269,7 +269,10 @@ __device__ __forceinline__ void tok_trig(const uint32_t* row32, int k, float& c,
 // Its slope is 1/(1 + en) above the edge and en/(1 + en) below, for both kinds.
 // In log2 units the exponent takes y as it is and the gate's kind is a factor,
 // not selects: the gated dQ pass at T=16384, H=8, lists of 14, one document
-// 508 -> 451 us, the error against fp64 as before.
+// 503 -> 448 us, the error against fp64 as before.  The backward adds the row's
+// softmax offset, the largest term, after slope and gate: first, as one fma less,
+// the pass took 446 us, but its coarser rounding put the fp32 gradients of slope,
+// δ and width 1% further from fp64.
 __device__ __forceinline__ float gate_y(float dd, float wd, float y_scale) { return (fabsf(dd) - wd) * y_scale; }
 __device__ __forceinline__ float gate_en(float y, float spw) { return spw * __builtin_amdgcn_exp2f(-fabsf(y)); }
 __device__ __forceinline__ float gate_g(float y, float en1) { return fmaxf(y, 0.f) + __builtin_amdgcn_logf(en1); }
